@@ -28,6 +28,15 @@ struct KParams {
     double pf_pmin[CMP_MAX_PHASES];    // phasic energy floors of the phasic Phase-Field formulation
 };
 
+// v[dir] of a short array for a direction that may be known only at run time (a dynamic index would send the
+// array to scratch memory); folds away for a constant dir.
+template <int DIM>
+__device__ __forceinline__ double pick(const double* v, int dir)
+{
+    const double a = v[0], b = v[1], c = v[DIM > 2 ? 2 : 0];   // read before the selection, for the same reason
+    return (dir == 0) ? a : ((DIM == 2 || dir == 1) ? b : c);
+}
+
 __device__ __forceinline__ double smin(double a, double b) { return (b < a) ? b : a; }  // std::min
 __device__ __forceinline__ double smax(double a, double b) { return (a < b) ? b : a; }  // std::max
 __device__ __forceinline__ double dsign(double x) { return (x > 0.0) ? 1.0 : ((x < 0.0) ? -1.0 : 0.0); }
@@ -315,7 +324,7 @@ __device__ __forceinline__ double weno5_side(double n, double S, double I1, unsi
 // each is two fused multiply-adds on a shared square; the value is f_c + (sum_k t_k (f_k - f_c)) / sum_k t_k,
 // one division a side. Against one side at a time with plain divisions and a branch per value (with the
 // rest of the face's arithmetic below in the same form): ten steps of 256^2 0.283 -> 0.208 ms, four of a
-// 75 x 61 x 50 level 0.715 -> 0.577 ms, five of the 512^2 three-phase level 0.980 -> 0.586 ms.
+// 75 x 61 x 50 level 0.715 -> 0.577 ms.
 __device__ __forceinline__ void weno5_pair(double v0, double v1, double v2, double v3, double v4, double v5,
                                            double& L, double& R, unsigned& out)
 {
@@ -366,6 +375,27 @@ __device__ __forceinline__ void weno5_faces(const S& s, double* LW, double* RW)
             RW[n] = weno5_general<-1>(s(1, n), s(2, n), s(3, n), s(4, n), s(5, n));
         }
     }
+}
+
+// One side at a time, for the N-phase model: face value sum_k w_k f_k. Fast path: with
+// t_k = d_k prod_{j != k} IS_j^2 the value is (sum_k t_k f_k) / sum_k t_k, taken when that sum lies well inside
+// the double range (no scaling, one division); constant data (all IS zero), extreme IS ratios, NaN and inf go
+// through weno5_weights.
+template <int FACE>
+__device__ __forceinline__ double weno5(double f_mm, double f_m, double f_c, double f_p, double f_pp)
+{
+    constexpr double d0 = (FACE == 1) ? 3.0 / 10.0 : 1.0 / 10.0;
+    constexpr double d2 = (FACE == 1) ? 1.0 / 10.0 : 3.0 / 10.0;
+    constexpr double d1 = 1.0 - d0 - d2;
+    double f[3], IS[3];
+    weno5_parts<FACE>(f_mm, f_m, f_c, f_p, f_pp, f, IS);
+    const double q01 = IS[0] * IS[1], q02 = IS[0] * IS[2], q12 = IS[1] * IS[2];
+    const double t0 = d0 * (q12 * q12), t1 = d1 * (q02 * q02), t2 = d2 * (q01 * q01);
+    const double S = (t0 + t1) + t2;
+    if (S > 1e-290 && S < 1e290) return quot_normal(t0 * f[0] + t1 * f[1] + t2 * f[2], S);
+    double w[3];
+    weno5_weights<FACE>(IS, w);
+    return w[0] * f[0] + w[1] * f[1] + w[2] * f[2];
 }
 
 // Slope_TVD + Reconstruction2Face_MUSCL_D + Reconstruction2Face_Linear
@@ -513,7 +543,7 @@ template <int DIM>
 __device__ __forceinline__ double hllc_half(const FaceSide<DIM>& s, int dir, double S, double Sb,
                                             double S_Star, double* F)
 {
-    const double V = s.W[2 + dir];
+    const double V = pick<DIM>(s.W + 2, dir);
     const double p = s.W[2 + DIM];
     const double inv = quot(1.0, S - S_Star);
     const double q = (S - V) * inv;
@@ -523,9 +553,9 @@ __device__ __forceinline__ double hllc_half(const FaceSide<DIM>& s, int dir, dou
     F[0] = s.W[0] * un;
     F[1] = s.W[1] * un;
     const double ru = s.rho * un;
+    const double pn = p + Sb * (qr * dS);
 #pragma unroll
-    for (int m = 0; m < DIM; ++m) F[2 + m] = s.W[2 + m] * ru;
-    F[2 + dir] += p + Sb * (qr * dS);
+    for (int m = 0; m < DIM; ++m) F[2 + m] = (m == dir) ? s.W[2 + m] * ru + pn : s.W[2 + m] * ru;
     F[2 + DIM] = (side_energy<DIM>(s) * un + p * V) + Sb * (dS * (qr * S_Star + p * inv));
     F[3 + DIM] = s.W[3 + DIM] * un;
     return un;
@@ -536,7 +566,7 @@ __device__ __forceinline__ double riemann(const FaceSide<DIM>& L, const FaceSide
                                           double* F, double& cmax)
 {
     constexpr int N = 4 + DIM;
-    const double VL = L.W[2 + dir], VR = R.W[2 + dir];
+    const double VL = pick<DIM>(L.W + 2, dir), VR = pick<DIM>(R.W + 2, dir);
     cmax = smax(L.c + sqrt_fast(L.q), R.c + sqrt_fast(R.q));
     if (RIEMANN == 2) {
         const double pL = L.W[2 + DIM], pR = R.W[2 + DIM];
@@ -635,7 +665,7 @@ __device__ __forceinline__ void recon_face_decided(const KParams& kp, int limite
     constexpr int N = 4 + DIM;
     constexpr int G = (SCHEME >= 5) ? 3 : (SCHEME == 1 ? 2 : 1);
     constexpr int IA = 3 + DIM;
-    const double dx = kp.dx[dir], idx = kp.inv_dx[dir];
+    const double dx = pick<DIM>(kp.dx, dir), idx = pick<DIM>(kp.inv_dx, dir);
     struct { double* W; } L{LW}, R{RW};
     bool done = false;
     if (THINC && (aL >= 0.0 || aR >= 0.0)) {
@@ -767,6 +797,31 @@ __device__ __forceinline__ void np_cons2prim(const KParams& kp, const double* U,
     W[I::E] = (rho_e - rho_D - BP) * (rho * inv);
 }
 
+// Primitive2Conservative (…Primitive2Conservative_Compressible5Eq_NPhase.H:15-62); AP, BP, rho out.
+template <int DIM, int NP>
+__device__ __forceinline__ void np_prim2cons(const KParams& kp, const double* W, double* U, double& AP,
+                                             double& BP, double& rho, int& bad)
+{
+    using I = NpIdx<DIM, NP>;
+    rho = W[0];
+#pragma unroll
+    for (int k = 1; k < NP; ++k) rho += W[k];
+    double ke = 0.0;
+#pragma unroll
+    for (int m = 0; m < DIM; ++m) {
+        U[I::MOM + m] = rho * W[I::MOM + m];
+        ke = (m == 0) ? W[I::MOM] * W[I::MOM] : ke + W[I::MOM + m] * W[I::MOM + m];
+    }
+    double rho_D;
+    np_mix<NP>(kp, W + I::A, W, AP, BP, rho_D, bad);
+#pragma unroll
+    for (int k = 0; k < NP; ++k) {
+        U[k] = W[k];
+        U[I::A + k] = W[I::A + k];
+    }
+    U[I::E] = (AP * W[I::E] + BP + rho_D) + (0.5 * rho) * ke;
+}
+
 // SoundSpeed with rho_c2_Phase / rho_c2_Mixture (…SoundSpeed_Compressible5Eq_NPhase.H:15-52,
 // …rho_c2_Mixture_Compressible5Eq_NPhase.H:15-52): K = 0 rho c^2 = sum_k alpha_k A_k rho_k c_k^2 / AP
 // with A_k rho_k c_k^2 = (A_k + 1) p + B_k; K = 1 Wood's 1/sum_k phi_k/(rho_k c_k^2).
@@ -835,102 +890,83 @@ __device__ __forceinline__ void np_limiter_consistent(const double* s, double* t
         for (int k = 0; k < NP; ++k) th[k] = 1.0;
         return;
     }
-    // to = clip(smx / smS, 0, 1), tm = clip(smS / smx, 0, 1): the smaller magnitude over the larger is
-    // the one quotient needed (the other is at least 1, or negative); smS = +0 leaves to the sign of smx
     const double smS = smx - S;
-    const bool less = fabs(smS) <= fabs(smx);
-    const double q = quot(less ? smS : smx, less ? smx : smS);
-    const double c = smax(smin(q, 1.0), 0.0);
-    const double o = ((smS == 0.0) ? smx > 0.0 : q > 0.0) ? 1.0 : 0.0;
-    const double to = less ? o : c, tm = less ? c : o;
+    const double to = smax(smin(quot(smx, smS), 1.0), 0.0);
+    const double tm = smax(smin(quot(smS, smx), 1.0), 0.0);
 #pragma unroll
     for (int k = 0; k < NP; ++k) th[k] = (k == imax) ? tm : to;
 }
 
 // FVM_Reconstruction2Face_Conservative_LimiterConsistent (…LimiterConsistent_Compressible5Eq_NPhase.H:15-73)
-// on a primitive face state W of the side whose cell primitives are c(n): the alpha_k rho_k and alpha_k
-// slopes to the face, theta from the alpha slopes, the linear face values with theta times the slope.
-// (The reference takes W to conservative and back first, which changes it by rounding alone.)
+// on a primitive face state W of the side whose cell primitives are c(n): prim->cons->prim as the
+// reference takes it, the alpha_k rho_k and alpha_k slopes to the face, theta from the alpha slopes,
+// the linear face values with theta times the slope.
 template <int DIM, int NP, typename C>
-__device__ __forceinline__ void np_limit_face(const KParams& kp, double* W, const C& c, double idx, int face,
+__device__ __forceinline__ void np_limit_face(const KParams& kp, double* W, const C& c, double dx, int face,
                                               int& bad)
 {
     using I = NpIdx<DIM, NP>;
-    double rho = W[0];
-#pragma unroll
-    for (int k = 1; k < NP; ++k) rho += W[k];
-    if (rho <= 0.0) bad = CMP_ERR_DENSITY;
-    if (kp.nasg) {
-        double AP, BP, rho_D;
-        np_mix<NP>(kp, W + I::A, W, AP, BP, rho_D, bad);
-    }
-    const double ih = double(face) * 2.0 * idx;
-    double dr[NP], da[NP], sa[NP], th[NP];
+    double U[I::N], AP, BP, rho;
+    np_prim2cons<DIM, NP>(kp, W, U, AP, BP, rho, bad);
+    np_cons2prim<DIM, NP>(kp, U, W, bad);
+    const double h = double(face) * 0.5 * dx, rh = rcp_refined(h);
+    double sr[NP], sa[NP], th[NP];
 #pragma unroll
     for (int k = 0; k < NP; ++k) {
-        dr[k] = W[k] - c(k);
-        da[k] = W[I::A + k] - c(I::A + k);
-        sa[k] = da[k] * ih;
+        sr[k] = quot_by(W[k] - c(k), h, rh);
+        sa[k] = quot_by(W[I::A + k] - c(I::A + k), h, rh);
     }
     np_limiter_consistent<NP>(sa, th);
 #pragma unroll
     for (int k = 0; k < NP; ++k) {
-        W[k] = c(k) + th[k] * dr[k];
-        W[I::A + k] = c(I::A + k) + th[k] * da[k];
+        W[k] = c(k) + double(face) * 0.5 * (th[k] * sr[k]) * dx;
+        W[I::A + k] = c(I::A + k) + double(face) * 0.5 * (th[k] * sa[k]) * dx;
     }
 }
 
 template <int DIM, int NP>
 struct FaceSideN {
     double W[NpIdx<DIM, NP>::N];
-    double rho, AP, BP, rho_D, q, c;    // q = |u|^2
+    double U[NpIdx<DIM, NP>::N];
+    double rho, AP, BP, c;
 };
 
 template <int DIM, int NP>
 __device__ __forceinline__ void np_make_side(const KParams& kp, FaceSideN<DIM, NP>& s, int& bad)
 {
     using I = NpIdx<DIM, NP>;
-    s.rho = s.W[0];
-#pragma unroll
-    for (int k = 1; k < NP; ++k) s.rho += s.W[k];
-#pragma unroll
-    for (int m = 0; m < DIM; ++m)
-        s.q = (m == 0) ? s.W[I::MOM] * s.W[I::MOM] : s.q + s.W[I::MOM + m] * s.W[I::MOM + m];
-    np_mix<NP>(kp, s.W + I::A, s.W, s.AP, s.BP, s.rho_D, bad);
+    np_prim2cons<DIM, NP>(kp, s.W, s.U, s.AP, s.BP, s.rho, bad);
     s.c = np_sound_speed<NP>(kp, s.W[I::E], s.W + I::A, s.W, s.rho, s.AP, bad);
 }
 
-template <int DIM, int NP>
-__device__ __forceinline__ double np_side_energy(const FaceSideN<DIM, NP>& s)
-{
-    return (s.AP * s.W[NpIdx<DIM, NP>::E] + s.BP + s.rho_D) + (0.5 * s.rho) * s.q;
-}
-
-// One side's HLLC flux (Riemann_HLLC …NPhase.H:16-162) with the star state of the side S* picks, in
-// hllc_half's form.
+// One side's HLLC flux (Riemann_HLLC …NPhase.H:16-162) with the star state of the side S* picks.
 template <int DIM, int NP>
 __device__ __forceinline__ double np_hllc_half(const FaceSideN<DIM, NP>& s, int dir, double S, double Sb,
                                                double S_Star, double* F)
 {
     using I = NpIdx<DIM, NP>;
-    const double V = s.W[I::MOM + dir];
+    const double V = pick<DIM>(s.W + I::MOM, dir);
     const double p = s.W[I::E];
     const double inv = quot(1.0, S - S_Star);
     const double q = (S - V) * inv;
-    const double un = V + Sb * (q - 1.0);
-    const double dS = S_Star - V;
-    const double qr = q * s.rho;
 #pragma unroll
     for (int k = 0; k < NP; ++k) {
-        F[k] = s.W[k] * un;
-        F[I::A + k] = s.W[I::A + k] * un;
+        F[k] = s.W[k] * V + Sb * (q * s.U[k] - s.U[k]);
+        F[I::A + k] = s.W[I::A + k] * V + Sb * (q * s.U[I::A + k] - s.U[I::A + k]);
     }
-    const double ru = s.rho * un;
 #pragma unroll
-    for (int m = 0; m < DIM; ++m) F[I::MOM + m] = s.W[I::MOM + m] * ru;
-    F[I::MOM + dir] += p + Sb * (qr * dS);
-    F[I::E] = (np_side_energy<DIM, NP>(s) * un + p * V) + Sb * (dS * (qr * S_Star + p * inv));
-    return un;
+    for (int m = 0; m < DIM; ++m) {
+        double Fm = s.U[I::MOM + m] * V;
+        double Cs = q * s.U[I::MOM + m];
+        if (m == dir) {
+            Fm += p;
+            Cs += q * s.rho * (S_Star - V);
+        }
+        F[I::MOM + m] = Fm + Sb * (Cs - s.U[I::MOM + m]);
+    }
+    const double CsE = q * s.U[I::E] + (S_Star - V) * (q * s.rho * S_Star + p * inv);
+    F[I::E] = (s.U[I::E] + p) * V + Sb * (CsE - s.U[I::E]);
+    return V + Sb * (q - 1.0);
 }
 
 // HLLC (RIEMANN 2) or HLL (1, Riemann_HLL …NPhase.H) of the N-phase model; returns u*_n.
@@ -940,16 +976,22 @@ __device__ __forceinline__ double np_riemann(const FaceSideN<DIM, NP>& L, const 
 {
     using I = NpIdx<DIM, NP>;
     constexpr int N = I::N;
-    const double VL = L.W[I::MOM + dir], VR = R.W[I::MOM + dir];
-    cmax = smax(L.c + sqrt_fast(L.q), R.c + sqrt_fast(R.q));
+    const double VL = pick<DIM>(L.W + I::MOM, dir), VR = pick<DIM>(R.W + I::MOM, dir);
+    double qL = 0.0, qR = 0.0;
+#pragma unroll
+    for (int m = 0; m < DIM; ++m) {
+        qL = (m == 0) ? L.W[I::MOM] * L.W[I::MOM] : qL + L.W[I::MOM + m] * L.W[I::MOM + m];
+        qR = (m == 0) ? R.W[I::MOM] * R.W[I::MOM] : qR + R.W[I::MOM + m] * R.W[I::MOM + m];
+    }
+    cmax = smax(L.c + sqrt_fast(qL), R.c + sqrt_fast(qR));
     const double pL = L.W[I::E], pR = R.W[I::E];
     if (RIEMANN == 2) {
         const double V_avg = 0.5 * (VL + VR);
         const double c_avg = 0.5 * (L.c + R.c);
-        const double SL = fmin(V_avg - c_avg, VL - L.c);
-        const double SR = fmax(V_avg + c_avg, VR + R.c);
-        const double mL = L.rho * (SL - VL), mR = R.rho * (SR - VR);
-        const double S_Star = quot(pR - pL + VL * mL - VR * mR, mL - mR);
+        const double SL = smin(V_avg - c_avg, VL - L.c);
+        const double SR = smax(V_avg + c_avg, VR + R.c);
+        const double S_Star = quot(pR - pL + L.rho * VL * (SL - VL) - R.rho * VR * (SR - VR),
+                                   L.rho * (SL - VL) - R.rho * (SR - VR));
         if (S_Star > 0.0) return np_hllc_half<DIM, NP>(L, dir, SL, smin(0.0, SL), S_Star, F);
         if (S_Star < 0.0) return np_hllc_half<DIM, NP>(R, dir, SR, smax(0.0, SR), S_Star, F);
         double FR_[N];
@@ -964,19 +1006,14 @@ __device__ __forceinline__ double np_riemann(const FaceSideN<DIM, NP>& L, const 
         const double inv = quot(1.0, Sp - Sm);
 #pragma unroll
         for (int n = 0; n < N; ++n) {
-            double UL, UR, FL, FR;
-            if (n < NP || n >= I::A) {
-                UL = L.W[n]; UR = R.W[n];
-                FL = UL * VL; FR = UR * VR;
-            } else if (n == I::E) {
-                UL = np_side_energy<DIM, NP>(L); UR = np_side_energy<DIM, NP>(R);
-                FL = (UL + pL) * VL; FR = (UR + pR) * VR;
-            } else {
-                UL = L.rho * L.W[n]; UR = R.rho * R.W[n];
-                FL = UL * VL + ((n == I::MOM + dir) ? pL : 0.0);
-                FR = UR * VR + ((n == I::MOM + dir) ? pR : 0.0);
+            double FL, FR;
+            if (n < NP || n >= I::A) { FL = L.W[n] * VL; FR = R.W[n] * VR; }
+            else if (n == I::E) { FL = (L.U[n] + pL) * VL; FR = (R.U[n] + pR) * VR; }
+            else {
+                FL = L.U[n] * VL + ((n == I::MOM + dir) ? pL : 0.0);
+                FR = R.U[n] * VR + ((n == I::MOM + dir) ? pR : 0.0);
             }
-            F[n] = (Sp * FL - Sm * FR + Sp * Sm * (UR - UL)) * inv;
+            F[n] = (Sp * FL - Sm * FR + Sp * Sm * (R.U[n] - L.U[n])) * inv;
         }
         return (Sp * VL - Sm * VR) * inv;
     }
@@ -990,19 +1027,24 @@ __device__ __forceinline__ void np_recon_face(const KParams& kp, int limiter, in
                                               double* RW, int& bad)
 {
     constexpr int N = NpIdx<DIM, NP>::N;
-    const double dx = kp.dx[dir], idx = kp.inv_dx[dir];
+    const double dx = pick<DIM>(kp.dx, dir), idx = pick<DIM>(kp.inv_dx, dir);
     if (SCHEME == 5) {
-        weno5_faces<0, N - 1>(s, LW, RW);
-        np_limit_face<DIM, NP>(kp, LW, [&](int n) { return s(2, n); }, idx, 1, bad);
-        np_limit_face<DIM, NP>(kp, RW, [&](int n) { return s(3, n); }, idx, -1, bad);
+#pragma unroll
+        for (int n = 0; n < N; ++n) {
+            const double v0 = s(0, n), v1 = s(1, n), v2 = s(2, n), v3 = s(3, n), v4 = s(4, n), v5 = s(5, n);
+            LW[n] = weno5<1>(v0, v1, v2, v3, v4);
+            RW[n] = weno5<-1>(v1, v2, v3, v4, v5);
+        }
+        np_limit_face<DIM, NP>(kp, LW, [&](int n) { return s(2, n); }, dx, 1, bad);
+        np_limit_face<DIM, NP>(kp, RW, [&](int n) { return s(3, n); }, dx, -1, bad);
     } else if (SCHEME == 1) {
 #pragma unroll
         for (int n = 0; n < N; ++n) {
             LW[n] = muscl(s(0, n), s(1, n), s(2, n), dx, idx, 1, limiter);
             RW[n] = muscl(s(1, n), s(2, n), s(3, n), dx, idx, -1, limiter);
         }
-        np_limit_face<DIM, NP>(kp, LW, [&](int n) { return s(1, n); }, idx, 1, bad);
-        np_limit_face<DIM, NP>(kp, RW, [&](int n) { return s(2, n); }, idx, -1, bad);
+        np_limit_face<DIM, NP>(kp, LW, [&](int n) { return s(1, n); }, dx, 1, bad);
+        np_limit_face<DIM, NP>(kp, RW, [&](int n) { return s(2, n); }, dx, -1, bad);
     } else {
 #pragma unroll
         for (int n = 0; n < N; ++n) {
@@ -1349,25 +1391,22 @@ template <int DIM, typename A>
 __device__ __forceinline__ double face_normal_component(const KParams& kp, int dir, const A& a)
 {
     const double fc = a(0, 0, 0), fm = a(-1, 0, 0);
-    const double gd = (fc - fm) * kp.inv_dx[dir];
+    const double gd = (fc - fm) * pick<DIM>(kp.inv_dx, dir);
     double sum = gd * gd;
-    int tdim[2] = {0, 0};
-    int nt = 0;
-#pragma unroll
-    for (int t = 0; t < DIM; ++t)
-        if (t != dir) tdim[nt++] = t;
 #pragma unroll
     for (int q = 0; q < DIM - 1; ++q) {
+        const int td = (dir <= q) ? q + 1 : q;   // the q-th direction other than dir
         double edge[2];
 #pragma unroll
         for (int sgn = 0; sgn < 2; ++sgn) {
             const int o = sgn ? 1 : -1;
             const double C = (q == 0) ? a(0, o, 0) : a(0, 0, o);
             const double D = (q == 0) ? a(-1, o, 0) : a(-1, 0, o);
-            edge[sgn] = (dir < tdim[q]) ? 0.25 * fc + 0.25 * fm + 0.25 * C + 0.25 * D
-                                        : 0.25 * fc + 0.25 * C + 0.25 * fm + 0.25 * D;
+            // the mean of the four cells around the edge, in ascending direction order
+            const double u = (dir < td) ? fm : C, v = (dir < td) ? C : fm;
+            edge[sgn] = 0.25 * fc + 0.25 * u + 0.25 * v + 0.25 * D;
         }
-        const double g = (edge[1] - edge[0]) * kp.inv_dx[tdim[q]];
+        const double g = (edge[1] - edge[0]) * pick<DIM>(kp.inv_dx, td);
         sum += g * g;
     }
     return (sum == 0.0) ? 0.0 : gd / sqrt(sum);

@@ -3,16 +3,17 @@
 // Built twice, with CMP_KERNEL_DIM=2 and CMP_KERNEL_DIM=3, so that the two dimensions compile in
 // parallel; cmp_capi.hip routes a call to the right instantiation.
 //
-// Stage kernel (one workgroup = one tile of a box):
-//   for each direction d:
-//     1. the primitives of the tile plus G cells on both sides along d are staged in LDS
-//        (cons->prim once per staged cell),
-//     2. every face of the tile along d is computed once, one face per thread (reconstruction,
-//        prim->cons, Riemann); flux and u*_n then go to LDS over the staged primitives,
-//     3. every cell accumulates (F_+ - F_-)/dx_d and (u*_+ - u*_-)/dx_d in registers;
-//   then dU = -div F, dU[alpha1] += phi1 (1+K1) div u*, and the RK3 combination writes the new
-//   state: dU never goes to HBM. The face wave speeds of the tile are max-reduced with wave
-//   shuffles and one 64-bit atomicMax per workgroup.
+// Stage kernel of the flow (k_stage; one workgroup = one tile of a box):
+//   1. the primitives of the tile and of the G cells beyond it on every side (a cross without corners)
+//      are staged in LDS, cons->prim once per staged cell;
+//   2. the faces of all directions form one list, dealt to the threads one after the other
+//      (reconstruction, prim->cons, Riemann; the direction is a run-time value); flux and u*_n then go
+//      to LDS over the staged primitives;
+//   3. every cell takes its flux differences: dU = -div F, dU[alpha1] += phi1 (1+K1) div u*, and the
+//      RK3 combination writes the new state: dU never goes to HBM. The face wave speeds of the tile are
+//      max-reduced with wave shuffles and one 64-bit atomicMax per workgroup.
+// The Phase-Field stage and the work-list kernel (tiles of run-time shape) go direction by direction: a
+// direction's staged cells, its faces, its flux differences accumulated in registers.
 #include "cmp_kernels.hpp"
 
 #ifndef CMP_KERNEL_DIM
@@ -21,8 +22,8 @@
 
 namespace cmp {
 
-// Tile shapes chosen so that every direction's face count fits one pass of the 256 threads:
-// 2D 16x15 (255 x-faces, 256 y-faces), 3D 8x8x3 (216, 216, 256).
+// Tile shapes: 2D 16x15 (255 x-faces, 256 y-faces), 3D 8x8x3 (216, 216, 256): every direction's faces fit
+// one pass of the 256 threads, and all of them together 511 and 688, which fill 8 and 10.75 waves.
 template <int DIM> struct Tile;
 template <> struct Tile<2> { static constexpr int X = 16, Y = 15, Z = 1; };
 template <> struct Tile<3> { static constexpr int X = 8, Y = 8, Z = 3; };
@@ -30,6 +31,25 @@ template <> struct Tile<3> { static constexpr int X = 8, Y = 8, Z = 3; };
 template <int SCHEME> struct Stencil { static constexpr int G = (SCHEME >= 5) ? 3 : (SCHEME == 1 ? 2 : 1); };
 
 constexpr int cmax3(int a, int b, int c) { return (a > b ? (a > c ? a : c) : (b > c ? b : c)); }
+
+// LDS layout of the flow's k_stage: the tile's cells, then per direction the 2 G layers beyond it (G below,
+// G above); strides are the full tile's whatever part of it the box fills. The faces' fluxes go over them.
+template <int DIM, int G>
+struct Cross {
+    static constexpr int TX = Tile<DIM>::X, TY = Tile<DIM>::Y, TZ = Tile<DIM>::Z;
+    static constexpr int CORE = TX * TY * TZ;
+    static constexpr int B0 = CORE, B1 = B0 + 2 * G * TY * TZ, B2 = B1 + 2 * G * TX * TZ;
+    static constexpr int CELLS = B2 + (DIM == 3 ? 2 * G * TX * TY : 0);
+    static constexpr int FACES = (TX + 1) * TY * TZ + TX * (TY + 1) * TZ + (DIM == 3 ? TX * TY * (TZ + 1) : 0);
+    static constexpr int RND = (FACES + NT - 1) / NT;   // faces a thread takes one after the other
+    static_assert(RND <= 3, "the kept fluxes are held in two register arrays");
+    template <int N> static constexpr int doubles()
+    {
+        return N * CELLS > (N + 1) * FACES ? N * CELLS : (N + 1) * FACES;
+    }
+    // alpha1 of the tile and one cell beyond it on every side, corners included (THINC's face normals)
+    static constexpr int AX = TX + 2, AY = TY + 2, ALPHAS = AX * AY * (DIM == 3 ? TZ + 2 : 1);
+};
 
 template <int DIM, int G>
 struct Lds {
@@ -40,7 +60,7 @@ struct Lds {
                                       DIM == 3 ? TX * TY * (TZ + 1) : 0);
 };
 
-// The tile shape the stage code is instantiated for. ShapeFixed: k_stage's one shape, whose
+// The tile shape the direction passes are instantiated for. ShapeFixed: the one shape above, whose
 // extents fold into the index arithmetic as constants. ShapeRT: a shape read per tile at run time
 // (k_stage_list), any TX x TY x TZ of at most NT cells whose staged region along every direction
 // fits LdsRT::RMAX cells and whose faces along every direction fit NT + LdsRT::XS (the faces beyond
@@ -107,6 +127,11 @@ __device__ __forceinline__ void split3(int r, int e0, int e1, float rcp0, float 
     }
 }
 
+__device__ __forceinline__ void split3(int r, int e0, int e1, int& x, int& y, int& z)
+{
+    split3<ShapeRT>(r, e0, e1, __builtin_amdgcn_rcpf((float)e0), __builtin_amdgcn_rcpf((float)(e0 * e1)), x, y, z);
+}
+
 // Maps a workgroup to a tile so that the workgroups one XCD receives (blocks b, b+8, b+16, ...
 // under round-robin dispatch) hold consecutive tiles, whose halos overlap in that XCD's L2.
 __device__ __forceinline__ int xcd_tile(int b, int nb)
@@ -115,13 +140,14 @@ __device__ __forceinline__ int xcd_tile(int b, int nb)
     return x * q + (x < r ? x : r) + (b >> 3);
 }
 
-// What one workgroup's direction passes share.
+// What the reads of one workgroup share.
 template <int DIM>
 struct StageCtx {
     const KParams& kp;
     int limiter;
     const BoxDev& bx;
     const double* __restrict__ Ub;
+    const double* __restrict__ Ut;   // the tile's lowest cell
     int tlo[3];
     int n[3];
     int tid, cx, cy, cz;
@@ -215,64 +241,115 @@ __device__ __noinline__ GhostSrc ghost_source(const FillDev* __restrict__ fd, in
     return g;
 }
 
-// A cell outside the tile's box, read as the ghost fill would write it (the box's own stale ghost
-// value when the fill has no source for it; the error is then reported as the fill reports it).
-template <int DIM, int N>
-__device__ __forceinline__ void read_ghost(const StageCtx<DIM>& cx_, int i, int j, int k, long long c, double* Uc,
-                                           int& bad)
-{
-    constexpr int MOM = (N == 4 + DIM) ? 2 : (N - DIM - 1) / 2;
-    const GhostSrc g = ghost_source<DIM>(cx_.fd, i, j, k);
-    if (g.err) {
-        bad = g.err;
-#pragma unroll
-        for (int q = 0; q < N; ++q) Uc[q] = cx_.Ub[c + q * cx_.bx.sn];
-        return;
-    }
-#pragma unroll
-    for (int q = 0; q < N; ++q) {
-        const double v = cx_.Ul[g.si + q * g.sn];
-        Uc[q] = (q >= MOM && q < MOM + DIM && ((g.flip >> (q - MOM)) & 1u)) ? -v : v;
-    }
-}
+// Where a staged cell's components are: the first one, the component stride, and the momenta to negate.
+struct CellSrc {
+    const double* p;
+    long long sn;
+    unsigned flip;
+};
 
 // A cell beyond the tile's box along D (side 0 low, 1 high) by the tile's halo source: a
 // neighbour box's cell (periodic image along D), the own box's boundary cell (clamp) or mirror
-// image (normal or all momenta negated), or the cell-by-cell lookup.
-template <int DIM, int N, int D>
-__device__ __forceinline__ void read_halo(const StageCtx<DIM>& cx_, int side, int i, int j, int k, long long c,
-                                          double* Uc, int& bad)
+// image (normal or all momenta negated), or the cell-by-cell lookup (the box's own stale ghost value
+// when the fill has no source for it; the error is then reported as the fill reports it).
+template <int DIM, int D>
+__device__ __forceinline__ CellSrc halo_source(const StageCtx<DIM>& cx_, int side, int i, int j, int k, int& bad)
 {
-    constexpr int MOM = (N == 4 + DIM) ? 2 : (N - DIM - 1) / 2;
-    const int code = cx_.halo[D][side];
+    const int lo_src = cx_.halo[D][0], hi_src = cx_.halo[D][1];
+    const int code = side ? hi_src : lo_src;
+    const BoxDev& bx = cx_.bx;
     int s[3] = {i, j, k};
     const int dlo = cx_.fd->dlo[D], dhi = cx_.fd->dhi[D];
     if (code >= 0) {
         const BoxDev& nb = cx_.boxes[code];
         if (s[D] < dlo) s[D] += dhi - dlo + 1;
         else if (s[D] > dhi) s[D] -= dhi - dlo + 1;
-        const double* __restrict__ src = cx_.Ul + nb.off + fab_index(nb, s[0], s[1], s[2]);
-        const long long sn = nb.sn;
-#pragma unroll
-        for (int q = 0; q < N; ++q) Uc[q] = src[q * sn];
-    } else if (code == HALO_LOOKUP) {
-        read_ghost<DIM, N>(cx_, i, j, k, c, Uc, bad);
-    } else {
-        if (code == HALO_CLAMP) s[D] = (s[D] < dlo) ? dlo : dhi;
-        else s[D] = (s[D] < dlo) ? 2 * dlo - 1 - s[D] : 2 * dhi + 1 - s[D];
-        const BoxDev& bx = cx_.bx;
-        const long long cc = fab_index(bx, s[0], s[1], s[2]);
-#pragma unroll
-        for (int q = 0; q < N; ++q) {
-            const double v = cx_.Ub[cc + q * bx.sn];
-            const bool neg = (code == HALO_MIRROR && q == MOM + D) ||
-                             (code == HALO_MIRROR_ALL && q >= MOM && q < MOM + DIM);
-            Uc[q] = neg ? -v : v;
-        }
+        // (a level's fabs have fewer than 2^31 cells, which level creation checks)
+        const int c = (s[0] - nb.flo[0]) + (int)nb.sj * (s[1] - nb.flo[1]) + (int)nb.sk * (s[2] - nb.flo[2]);
+        return {cx_.Ul + nb.off + c, nb.sn, 0u};
     }
+    if (code == HALO_LOOKUP) {
+        const GhostSrc g = ghost_source<DIM>(cx_.fd, i, j, k);
+        if (g.err == 0) return {cx_.Ul + g.si, g.sn, g.flip};
+        bad = g.err;
+        return {cx_.Ub + fab_index(bx, i, j, k), bx.sn, 0u};
+    }
+    if (code == HALO_CLAMP) s[D] = (s[D] < dlo) ? dlo : dhi;
+    else s[D] = (s[D] < dlo) ? 2 * dlo - 1 - s[D] : 2 * dhi + 1 - s[D];
+    return {cx_.Ub + fab_index(bx, s[0], s[1], s[2]), bx.sn,
+            (code == HALO_MIRROR) ? (1u << D) : (code == HALO_MIRROR_ALL) ? ((1u << DIM) - 1u) : 0u};
 }
 
-// One direction of the stage kernel (D known at compile time): stage the primitives of the tile
+// The source of cell (i, j, k) of the tile or of its layers beyond direction D.
+template <int DIM, int D>
+__device__ __forceinline__ CellSrc cell_source(const StageCtx<DIM>& cx_, int i, int j, int k, int& bad)
+{
+    const BoxDev& bx = cx_.bx;
+    const int cd = (D == 0) ? i : ((D == 1) ? j : k);
+    if (cx_.fd && (cd < bx.lo[D] || cd > bx.hi[D]))
+        return halo_source<DIM, D>(cx_, cd > bx.hi[D] ? 1 : 0, i, j, k, bad);
+    // (from the tile's first cell a cell of the tile or its layers is a few rows or planes away: 32 bits)
+    const int rel = (i - cx_.tlo[0]) + (int)bx.sj * (j - cx_.tlo[1]) + (int)bx.sk * (k - cx_.tlo[2]);
+    return {cx_.Ut + rel, bx.sn, 0u};
+}
+
+// A staged cell: its components from their source, then its primitives into its LDS slot (component stride
+// `stride`).
+template <int DIM, int NP>
+__device__ __forceinline__ void load_cell(const CellSrc& src, double* Uc)
+{
+    constexpr int N = NP ? 2 * NP + DIM + 1 : 4 + DIM;
+#pragma unroll
+    for (int q = 0; q < N; ++q) Uc[q] = src.p[q * src.sn];
+}
+template <int DIM, int NP>
+__device__ __forceinline__ void stage_cell(const KParams& kp, double* Uc, unsigned flip, double* slot, int stride, int& bad)
+{
+    constexpr int N = NP ? 2 * NP + DIM + 1 : 4 + DIM;
+    constexpr int MOM = NP ? NP : 2;
+    double Wc[N];
+#pragma unroll
+    for (int m = 0; m < DIM; ++m)
+        if ((flip >> m) & 1u) Uc[MOM + m] = -Uc[MOM + m];
+    if constexpr (NP > 0)
+        np_cons2prim<DIM, (NP > 0 ? NP : 2)>(kp, Uc, Wc, bad);
+    else
+        cons2prim<DIM>(kp, Uc, Wc, bad);
+#pragma unroll
+    for (int q = 0; q < N; ++q) slot[q * stride] = Wc[q];
+}
+
+// alpha1 at a cell next to the tile for THINC's face normals, read from the state itself, which the staging
+// has just brought into L2 (the transverse neighbours of the layers are not staged).
+template <int DIM>
+__device__ __forceinline__ double alpha_at(const StageCtx<DIM>& cx_, int pi, int pj, int pk, int& bad)
+{
+    const BoxDev& bx = cx_.bx;
+    if (cx_.fd && (pi < bx.lo[0] || pi > bx.hi[0] || pj < bx.lo[1] || pj > bx.hi[1] ||
+                   (DIM == 3 && (pk < bx.lo[2] || pk > bx.hi[2])))) {
+        const GhostSrc gs = ghost_source<DIM>(cx_.fd, pi, pj, pk);
+        if (gs.err == 0) return cx_.Ul[gs.si + (3 + DIM) * gs.sn];
+        bad = gs.err;
+    }
+    return cx_.Ub[fab_index(bx, pi, pj, pk) + (3 + DIM) * bx.sn];
+}
+
+// The component along D of the face normal at the face below cell (ci, cj, ck).
+template <int DIM, int D>
+__device__ __forceinline__ double normal_at(const StageCtx<DIM>& cx_, int ci, int cj, int ck, int& bad)
+{
+    auto aa = [&](int od, int o1, int o2) -> double {
+        const int lo = (od == -1) ? 1 : 0;
+        int pi = ci - (D == 0 ? lo : 0), pj = cj - (D == 1 ? lo : 0), pk = ck - (D == 2 ? lo : 0);
+        if (D == 0) { pj += o1; pk += (DIM == 3) ? o2 : 0; }
+        else if (D == 1) { pi += o1; pk += (DIM == 3) ? o2 : 0; }
+        else { pi += o1; pj += o2; }
+        return alpha_at<DIM>(cx_, pi, pj, pk, bad);
+    };
+    return face_normal_component<DIM>(cx_.kp, D, aa);
+}
+
+// One direction of a tile (D known at compile time): stage the primitives of the tile
 // plus G cells on both sides along D, compute every face along D once, and accumulate the flux and
 // u*_n differences of the thread's cell. sh: the tile shape; sW / sF: the staged primitives and,
 // over them, the fluxes of the first NT faces; sX: the fluxes of the faces beyond NT.
@@ -346,24 +423,11 @@ __device__ __forceinline__ void dir_pass(const StageCtx<DIM>& cx_, const SH& sh,
         int x, y, z;
         split3<SH>(r, E0, E1, rE0, rE01, x, y, z);
         if (x >= e0 || y >= e1 || z >= e2) continue;
-        const int i = cx_.tlo[0] + x - (D == 0 ? G : 0);
-        const int j = cx_.tlo[1] + y - (D == 1 ? G : 0);
-        const int k = cx_.tlo[2] + z - (D == 2 ? G : 0);
-        const long long c = fab_index(bx, i, j, k);
-        double Uc[N], Wc[N];
-        const int cd = (D == 0) ? i : ((D == 1) ? j : k);
-        if (cx_.fd && (cd < bx.lo[D] || cd > bx.hi[D])) {
-            read_halo<DIM, N, D>(cx_, cd > bx.hi[D] ? 1 : 0, i, j, k, c, Uc, bad);
-        } else {
-#pragma unroll
-            for (int q = 0; q < N; ++q) Uc[q] = cx_.Ub[c + q * bx.sn];
-        }
-        if constexpr (NP > 0)
-            np_cons2prim<DIM, NP>(kp, Uc, Wc, bad);
-        else
-            cons2prim<DIM>(kp, Uc, Wc, bad);
-#pragma unroll
-        for (int q = 0; q < N; ++q) sW[q * RMAX + r] = Wc[q];
+        const CellSrc src = cell_source<DIM, D>(cx_, cx_.tlo[0] + x - (D == 0 ? G : 0), cx_.tlo[1] + y - (D == 1 ? G : 0),
+                                                cx_.tlo[2] + z - (D == 2 ? G : 0), bad);
+        double Uc[N];
+        load_cell<DIM, NP>(src, Uc);
+        stage_cell<DIM, NP>(kp, Uc, src.flip, sW + r, RMAX, bad);
     }
     __syncthreads();
     // 2. faces along D: one face per thread and pass (the fixed shape has at most NT faces per
@@ -413,33 +477,11 @@ __device__ __forceinline__ void dir_pass(const StageCtx<DIM>& cx_, const SH& sh,
                 cmax_loc = smax(cmax_loc, c);
             }
         } else {
-            double aL = -1.0, aR = -1.0;
-            if constexpr (THINC) {
-                // THINC decision (gates, face normal, tanh profile) ahead of the base reconstruction.
-                // The face normal is needed only where the volume-fraction gates admit THINC, so its
-                // alpha1 stencil (the face's two cells and their transverse neighbours, transverse
-                // axes in ascending order) is read from the state itself, which the staging pass has
-                // just brought into L2, instead of being staged for every face.
-                const int hi_ = cx_.tlo[0] + x, hj = cx_.tlo[1] + y, hk = cx_.tlo[2] + ((DIM == 3) ? z : 0);
-                auto aa = [&](int od, int o1, int o2) -> double {
-                    const int lo = (od == -1) ? 1 : 0;
-                    int pi = hi_ - (D == 0 ? lo : 0), pj = hj - (D == 1 ? lo : 0), pk = hk - (D == 2 ? lo : 0);
-                    if (D == 0) { pj += o1; pk += (DIM == 3) ? o2 : 0; }
-                    else if (D == 1) { pi += o1; pk += (DIM == 3) ? o2 : 0; }
-                    else { pi += o1; pj += o2; }
-                    if (cx_.fd && (pi < bx.lo[0] || pi > bx.hi[0] || pj < bx.lo[1] || pj > bx.hi[1] ||
-                                   (DIM == 3 && (pk < bx.lo[2] || pk > bx.hi[2])))) {
-                        const GhostSrc gs = ghost_source<DIM>(cx_.fd, pi, pj, pk);
-                        if (gs.err == 0) return cx_.Ul[gs.si + (3 + DIM) * gs.sn];
-                        bad = gs.err;
-                    }
-                    return cx_.Ub[fab_index(bx, pi, pj, pk) + (3 + DIM) * bx.sn];
-                };
-                auto normal = [&]() -> double { return face_normal_component<DIM>(kp, D, aa); };
-                thinc_decide<DIM, G>(kp, st, normal, aL, aR);
-            }
+            auto normal = [&]() -> double {
+                return normal_at<DIM, D>(cx_, cx_.tlo[0] + x, cx_.tlo[1] + y, cx_.tlo[2] + ((DIM == 3) ? z : 0), bad);
+            };
             double c;
-            un = face_flux_decided<DIM, SCHEME, RIEMANN, THINC>(kp, cx_.limiter, D, st, aL, aR, Fl, c, bad);
+            un = face_flux<DIM, SCHEME, RIEMANN, THINC>(kp, cx_.limiter, D, st, normal, Fl, c, bad);
             if (a < cx_.n[D]) {
                 if (__builtin_isnan(c)) bad = CMP_ERR_NAN;
                 cmax_loc = smax(cmax_loc, c);
@@ -485,153 +527,405 @@ __device__ __forceinline__ void dir_pass(const StageCtx<DIM>& cx_, const SH& sh,
     __syncthreads();
 }
 
-// Minimum resident waves per SIMD the register allocator must leave room for (0: compiler's choice).
-#ifndef CMP_STAGE_WAVES
-#define CMP_STAGE_WAVES 2
-#endif
-#if CMP_STAGE_WAVES > 0
-#define CMP_STAGE_ATTR __attribute__((amdgpu_waves_per_eu(CMP_STAGE_WAVES)))
-#else
-#define CMP_STAGE_ATTR
-#endif
-
-// The stage of one tile (box bx, lowest cell tlo, shape sh, halo sources halo): staging, faces and
-// flux differences per direction, then the cell update of `mode`; c_max max-accumulated into
-// *cmax_bits, the error word into *err. sWF / sRed: the workgroup's LDS (sWF: lds_doubles of the
-// shape policy's layout).
-template <int DIM, int SCHEME, int RIEMANN, bool THINC, int NP, class SH>
-__device__ __forceinline__ void stage_tile(const KParams& kp, int limiter, int mode, int stage, const BoxDev& bx,
-                                           const int* tlo, const SH& sh, const int (&halo)[3][2],
-                                           const BoxDev* __restrict__ boxes,
-                                           const double* __restrict__ Us, const double* Un, double* Uout,
-                                           const double* __restrict__ dtp, unsigned long long* cmax_bits, int* err,
-                                           const double* __restrict__ gq, const FillDev* __restrict__ fd,
-                                           double* sWF, double* sRed, int tid = -1)
+// The cell update of `mode` from the flux differences acc and div u*: (i, j, k) a valid cell of box bx.
+template <int DIM, int SCHEME, int RIEMANN, int NP>
+__device__ __forceinline__ void update_cell(const KParams& kp, int mode, int stage, const BoxDev& bx, int i, int j, int k,
+                                            const double* acc, double divu, const double* __restrict__ Ub,
+                                            const double* Un, double* Uout, const double* __restrict__ dtp, int& bad)
 {
     constexpr int N = NP ? 2 * NP + DIM + 1 : 4 + DIM;
     constexpr int IA = 3 + DIM;
-    constexpr int G = Stencil<SCHEME>::G;
-    using LO = LdsOf<DIM, G, SH>;
-    double* const sW = sWF;
-    double* const sF = sWF;
-    double* const sX = sWF + (lds_doubles<N, LO>() - (N + 1) * LO::XS);
+    const long long c = fab_index(bx, i, j, k);
+    double Uc[N], dU[N];
+#pragma unroll
+    for (int q = 0; q < N; ++q) Uc[q] = Ub[c + q * bx.sn];
+    if constexpr (RIEMANN >= RIEMANN_PF_MIX) {
+        // faces hold fhat and the reference stores -fhat: -div(-fhat) = +div(fhat); the
+        // five-equation Phase-Field NC term is empty
+#pragma unroll
+        for (int q = 0; q < N; ++q) dU[q] = acc[q];
+    } else {
+#pragma unroll
+        for (int q = 0; q < N; ++q) dU[q] = -acc[q];
+        if constexpr (NP > 0) {
+            // every alpha_k takes phi_k (1 + K_k) div u* (…FVM_SurfaceIntegralNC_Compressible5Eq_NPhase.H)
+            double f[NP > 0 ? NP : 1];
+            np_nc_coefficients<DIM, (NP > 0 ? NP : 2)>(kp, Uc, f, bad);
+#pragma unroll
+            for (int m = 0; m < NP; ++m) dU[NpIdx<DIM, (NP > 0 ? NP : 2)>::A + m] += f[m] * divu;
+        } else {
+            dU[IA] += nc_coefficient<DIM>(kp, Uc, bad) * divu;
+        }
+    }
+    if (mode == MODE_RK) {
+        const double dt = *dtp;
+        double* Ob = Uout + bx.off;
+        const double* Nb = Un + bx.off;
+        if (stage == 0) {
+#pragma unroll
+            for (int q = 0; q < N; ++q) {
+                const double v = Uc[q] + dt * dU[q];
+                if (__builtin_isnan(v)) bad = CMP_ERR_NAN;
+                Ob[c + q * bx.sn] = v;
+            }
+        } else {
+            const double a = (stage == 1) ? 0.25 : (2.0 / 3.0);
+            const double b = (stage == 1) ? 0.75 : (1.0 / 3.0);
+            const double w = (stage == 1) ? 0.25 * dt : (2.0 / 3.0) * dt;
+#pragma unroll
+            for (int q = 0; q < N; ++q) {
+                const double v = (a * Uc[q] + b * Nb[c + q * bx.sn]) + w * dU[q];
+                if (__builtin_isnan(v)) bad = CMP_ERR_NAN;
+                Ob[c + q * bx.sn] = v;
+            }
+        }
+        if constexpr (SCHEME == 6 && NP == 0 && RIEMANN < RIEMANN_PF_MIX) {
+            // the bounded limiter keeps alpha1 in [0, 1]; a stage state beyond it (by more than
+            // rounding) is reported
+            const double an = Ob[c + IA * bx.sn];
+            if (an < -1.0e-12 || an > 1.0 + 1.0e-12) bad = CMP_ERR_ALPHA;
+        }
+    } else if (mode == MODE_RHS) {
+        const long long o = bx.ooff + (long long)(i - bx.olo[0]) + bx.osj * (j - bx.olo[1]) + bx.osk * (k - bx.olo[2]);
+#pragma unroll
+        for (int q = 0; q < N; ++q) Uout[o + q * bx.osn] = dU[q];
+    }
+}
 
-    if (tid < 0) tid = threadIdx.x;
+// The workgroup's wave speed into *cmax_bits (sRed: one double a wave).
+__device__ __forceinline__ void reduce_cmax(double cmax_loc, unsigned long long* cmax_bits, double* sRed, int tid)
+{
+    const double m = wave_max(cmax_loc);
+    if ((tid & 63) == 0) sRed[tid >> 6] = m;
+    __syncthreads();
+    if (tid == 0) {
+        double v = sRed[0];
+#pragma unroll
+        for (int w = 1; w < NT / 64; ++w) v = smax(v, sRed[w]);
+        // non-negative doubles order like their bit patterns; skip the atomic when the
+        // stored maximum is already as large
+        const unsigned long long vb = (unsigned long long)__double_as_longlong(v);
+        if (vb > __hip_atomic_load(cmax_bits, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
+            atomicMax(cmax_bits, vb);
+    }
+}
+
+// The stage of one tile, direction by direction (box bx, lowest cell tlo, shape sh, halo sources halo):
+// staging, faces and flux differences per direction, then the cell update of `mode`; c_max max-accumulated
+// into *cmax_bits, the error word into *err. sWF / sRed: the workgroup's LDS (sWF: lds_doubles of the
+// shape policy's layout).
+template <int DIM, int SCHEME, int RIEMANN, bool THINC, int NP, class SH>
+__device__ __forceinline__ void pass_tile(const KParams& kp, int limiter, int mode, int stage, const BoxDev& bx,
+                                          const int* tlo, const SH& sh, const int (&halo)[3][2],
+                                          const BoxDev* __restrict__ boxes,
+                                          const double* __restrict__ Us, const double* Un, double* Uout,
+                                          const double* __restrict__ dtp, unsigned long long* cmax_bits, int* err,
+                                          const double* __restrict__ gq, const FillDev* __restrict__ fd,
+                                          double* sWF, double* sRed)
+{
+    constexpr int N = NP ? 2 * NP + DIM + 1 : 4 + DIM;
+    using LO = LdsOf<DIM, Stencil<SCHEME>::G, SH>;
+    double* const sX = sWF + (lds_doubles<N, LO>() - (N + 1) * LO::XS);
+    const int tid = threadIdx.x;
     const int TX = sh.t(0), TY = sh.t(1), TZ = sh.t(2);
     int n[3];
     n[0] = min(TX, bx.hi[0] - tlo[0] + 1);
     n[1] = min(TY, bx.hi[1] - tlo[1] + 1);
     n[2] = (DIM == 3) ? min(TZ, bx.hi[2] - tlo[2] + 1) : 1;
-
     int cx, cy, cz;
-    if constexpr (SH::RT)
-        split3<SH>(tid, TX, TY, __builtin_amdgcn_rcpf((float)TX), __builtin_amdgcn_rcpf((float)(TX * TY)), cx, cy, cz);
-    else
-        split3<SH>(tid, TX, TY, 0.f, 0.f, cx, cy, cz);
+    if constexpr (SH::RT) split3(tid, TX, TY, cx, cy, cz);
+    else split3<SH>(tid, TX, TY, 0.f, 0.f, cx, cy, cz);
     const bool valid = (cx < n[0]) && (cy < n[1]) && (cz < n[2]);
     const double* __restrict__ Ub = Us + bx.off;
-
     int bad = 0;
     double cmax_loc = 0.0;
     double acc[N];
     double divu = 0.0;
 #pragma unroll
     for (int q = 0; q < N; ++q) acc[q] = 0.0;
-
-    StageCtx<DIM> ctx{kp, limiter, bx, Ub, {tlo[0], tlo[1], tlo[2]}, {n[0], n[1], n[2]}, tid, cx, cy, cz,
+    StageCtx<DIM> ctx{kp, limiter, bx, Ub, Ub + fab_index(bx, tlo[0], tlo[1], tlo[2]), {tlo[0], tlo[1], tlo[2]}, {n[0], n[1], n[2]}, tid, cx, cy, cz,
                       valid, gq, fd, Us, boxes,
                       {{halo[0][0], halo[0][1]}, {halo[1][0], halo[1][1]}, {halo[2][0], halo[2][1]}}};
-    dir_pass<DIM, SCHEME, RIEMANN, THINC, 0, NP>(ctx, sh, sW, sF, sX, acc, divu, cmax_loc, bad);
-    if (DIM > 1) dir_pass<DIM, SCHEME, RIEMANN, THINC, 1, NP>(ctx, sh, sW, sF, sX, acc, divu, cmax_loc, bad);
+    dir_pass<DIM, SCHEME, RIEMANN, THINC, 0, NP>(ctx, sh, sWF, sWF, sX, acc, divu, cmax_loc, bad);
+    if (DIM > 1) dir_pass<DIM, SCHEME, RIEMANN, THINC, 1, NP>(ctx, sh, sWF, sWF, sX, acc, divu, cmax_loc, bad);
     if (DIM > 2)
-        dir_pass<DIM, SCHEME, RIEMANN, THINC, (DIM > 2 ? 2 : 1), NP>(ctx, sh, sW, sF, sX, acc, divu, cmax_loc, bad);
-
-    if (valid) {
-        const int i = tlo[0] + cx, j = tlo[1] + cy, k = tlo[2] + cz;
-        const long long c = fab_index(bx, i, j, k);
-        double Uc[N], dU[N];
-        if constexpr (RIEMANN >= RIEMANN_PF_MIX) {
-            // faces hold fhat and the reference stores -fhat: -div(-fhat) = +div(fhat); the
-            // five-equation Phase-Field NC term is empty
-#pragma unroll
-            for (int q = 0; q < N; ++q) {
-                Uc[q] = Ub[c + q * bx.sn];
-                dU[q] = acc[q];
-            }
-        } else if constexpr (NP > 0) {
-            // every alpha_k takes phi_k (1 + K_k) div u* (…FVM_SurfaceIntegralNC_Compressible5Eq_NPhase.H)
-#pragma unroll
-            for (int q = 0; q < N; ++q) {
-                Uc[q] = Ub[c + q * bx.sn];
-                dU[q] = -acc[q];
-            }
-            double f[NP > 0 ? NP : 1];
-            np_nc_coefficients<DIM, NP>(kp, Uc, f, bad);
-#pragma unroll
-            for (int k = 0; k < NP; ++k) dU[NpIdx<DIM, NP>::A + k] += f[k] * divu;
-        } else {
-#pragma unroll
-            for (int q = 0; q < N; ++q) {
-                Uc[q] = Ub[c + q * bx.sn];
-                dU[q] = -acc[q];
-            }
-            dU[IA] += nc_coefficient<DIM>(kp, Uc, bad) * divu;
-        }
-        if (mode == MODE_RK) {
-            const double dt = *dtp;
-            double* Ob = Uout + bx.off;
-            const double* Nb = Un + bx.off;
-            if (stage == 0) {
-#pragma unroll
-                for (int q = 0; q < N; ++q) {
-                    const double v = Uc[q] + dt * dU[q];
-                    if (__builtin_isnan(v)) bad = CMP_ERR_NAN;
-                    Ob[c + q * bx.sn] = v;
-                }
-            } else {
-                const double a = (stage == 1) ? 0.25 : (2.0 / 3.0);
-                const double b = (stage == 1) ? 0.75 : (1.0 / 3.0);
-                const double w = (stage == 1) ? 0.25 * dt : (2.0 / 3.0) * dt;
-#pragma unroll
-                for (int q = 0; q < N; ++q) {
-                    const double v = (a * Uc[q] + b * Nb[c + q * bx.sn]) + w * dU[q];
-                    if (__builtin_isnan(v)) bad = CMP_ERR_NAN;
-                    Ob[c + q * bx.sn] = v;
-                }
-            }
-            if constexpr (SCHEME == 6 && NP == 0 && RIEMANN < RIEMANN_PF_MIX) {
-                // the bounded limiter keeps alpha1 in [0, 1]; a stage state beyond it (by more than
-                // rounding) is reported
-                const double an = Ob[c + IA * bx.sn];
-                if (an < -1.0e-12 || an > 1.0 + 1.0e-12) bad = CMP_ERR_ALPHA;
-            }
-        } else if (mode == MODE_RHS) {
-            const long long o = bx.ooff + (long long)(i - bx.olo[0]) + bx.osj * (j - bx.olo[1]) + bx.osk * (k - bx.olo[2]);
-#pragma unroll
-            for (int q = 0; q < N; ++q) Uout[o + q * bx.osn] = dU[q];
-        }
-    }
-
-    if (cmax_bits) {
-        const double m = wave_max(cmax_loc);
-        if ((tid & 63) == 0) sRed[tid >> 6] = m;
-        __syncthreads();
-        if (tid == 0) {
-            double v = sRed[0];
-#pragma unroll
-            for (int w = 1; w < NT / 64; ++w) v = smax(v, sRed[w]);
-            // non-negative doubles order like their bit patterns; skip the atomic when the
-            // stored maximum is already as large
-            const unsigned long long vb = (unsigned long long)__double_as_longlong(v);
-            if (vb > __hip_atomic_load(cmax_bits, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
-                atomicMax(cmax_bits, vb);
-        }
-    }
+        dir_pass<DIM, SCHEME, RIEMANN, THINC, (DIM > 2 ? 2 : 1), NP>(ctx, sh, sWF, sWF, sX, acc, divu, cmax_loc, bad);
+    if (valid)
+        update_cell<DIM, SCHEME, RIEMANN, NP>(kp, mode, stage, bx, tlo[0] + cx, tlo[1] + cy, tlo[2] + cz, acc, divu, Ub,
+                                              Un, Uout, dtp, bad);
+    if (cmax_bits) reduce_cmax(cmax_loc, cmax_bits, sRed, tid);
     if (bad && err) atomicMax(err, bad);
 }
 
+// The flow stage of one tile (box bx, lowest cell tlo, halo sources halo): the cross of primitives, the faces
+// of every direction in one list, the cell update of `mode`; c_max max-accumulated into *cmax_bits, the error
+// word into *err. sWF / sA / sRed: the workgroup's LDS (sA: THINC only).
+// Bound by FP64 issue (81% of the cycles on a 256^3 level). Against the direction passes above, a 3D tile
+// stages 864 cells instead of 1248, waits at 4 barriers instead of 12, and its 688 faces fill 10.75 waves
+// instead of 12; a clipped tile's faces fill as many waves as it has faces. Same boxes, before and after, on
+// one card: ten steps of 256^2 208 -> 190 us, five of 1024 x 256 with WENO5B 694 -> 544, four of a ragged
+// 75 x 61 x 50 level 577 -> 467, 24 served cases 781 -> 675; the 256^3 droplet's stage with THINC 2.94 -> 2.83
+// ms, without 2.71 -> 2.50.
+// Larger tiles (8x8x4, 16x16 in 7 to 16 waves) measured slower: fewer workgroups a CU, so that their loads and
+// barriers have less arithmetic of others to hide behind, and waves unevenly spread over the SIMDs.
 template <int DIM, int SCHEME, int RIEMANN, bool THINC, int NP>
-__global__ __launch_bounds__(NT) CMP_STAGE_ATTR
+__device__ __forceinline__ void flow_tile(const KParams& kp, int limiter, int mode, int stage, const BoxDev& bx,
+                                          const int* tlo, const int (&halo)[3][2], const BoxDev* __restrict__ boxes,
+                                          const double* __restrict__ Us, const double* Un, double* Uout,
+                                          const double* __restrict__ dtp, unsigned long long* cmax_bits, int* err,
+                                          const FillDev* __restrict__ fd, double* sWF, double* sA, double* sRed)
+{
+    constexpr int N = NP ? 2 * NP + DIM + 1 : 4 + DIM;
+    constexpr int IA = 3 + DIM;
+    constexpr int G = Stencil<SCHEME>::G;
+    using C = Cross<DIM, G>;
+    constexpr int TX = C::TX, TY = C::TY, RND = C::RND;
+    const int tid = threadIdx.x;
+    const int n0 = min(C::TX, bx.hi[0] - tlo[0] + 1), n1 = min(C::TY, bx.hi[1] - tlo[1] + 1);
+    const int n2 = (DIM == 3) ? min(C::TZ, bx.hi[2] - tlo[2] + 1) : 1;
+    const int nc = n0 * n1 * n2;
+    const double* __restrict__ Ub = Us + bx.off;
+    int bad = 0;
+    double cmax_loc = 0.0;
+    StageCtx<DIM> ctx{kp, limiter, bx, Ub, Ub + fab_index(bx, tlo[0], tlo[1], tlo[2]), {tlo[0], tlo[1], tlo[2]}, {n0, n1, n2}, tid, 0, 0, 0, true, nullptr, fd, Us,
+                      boxes, {{halo[0][0], halo[0][1]}, {halo[1][0], halo[1][1]}, {halo[2][0], halo[2][1]}}};
+
+    // 1. the cross of primitives: every load of the thread's cells first, then their primitives (a large
+    // state's loads come from HBM, one latency for all of them instead of one a cell). The tile's cells and the
+    // layers of each direction are dealt one after the other, each starting at the wave after the last one's, so
+    // that the waves share them evenly and a wave runs one kind of source at a time.
+    constexpr int CW = (C::CORE + 63) / 64 * 64, W0 = (C::B1 - C::B0 + 63) / 64 * 64, W1 = (C::B2 - C::B1 + 63) / 64 * 64;
+    constexpr int IT0 = (W0 + NT - 1) / NT, IT1 = (W1 + NT - 1) / NT;
+    constexpr int IT2 = (DIM == 3) ? (C::CELLS - C::B2 + NT - 1) / NT : 0, IT = 1 + IT0 + IT1 + IT2;
+    static_assert(C::CORE <= NT, "one thread a cell");
+    const int h0 = 2 * G * n1 * n2, h1 = n0 * 2 * G * n2, h2 = (DIM == 3) ? n0 * n1 * 2 * G : 0;
+    double Uc[IT][N];
+    int slot[IT], mixed = 0;
+    unsigned flip[IT];
+    int cx, cy, cz;
+    split3(tid, n0, n1, cx, cy, cz);
+    const bool valid = tid < nc;
+    const unsigned cell = (unsigned)(cx + (int)bx.sj * cy + (int)bx.sk * cz);
+    slot[0] = -1;
+    flip[0] = 0u;
+    if (valid) {
+        slot[0] = cx + TX * (cy + TY * cz);
+#pragma unroll
+        for (int q = 0; q < N; ++q) Uc[0][q] = (ctx.Ut + q * bx.sn)[cell];
+    }
+#pragma unroll
+    for (int it = 0; it < IT0; ++it) {
+        const int r = it * NT + ((tid - CW) & (NT - 1)), o = 1 + it;
+        slot[o] = -1;
+        if (r < h0) {
+            int x, y, z;
+            split3(r, 2 * G, n1, x, y, z);
+            slot[o] = C::B0 + x + 2 * G * (y + TY * z);
+            const CellSrc src = cell_source<DIM, 0>(ctx, tlo[0] + (x < G ? x - G : n0 + x - G), tlo[1] + y, tlo[2] + z, bad);
+            load_cell<DIM, NP>(src, Uc[o]);
+            flip[o] = src.flip;
+        }
+    }
+#pragma unroll
+    for (int it = 0; it < IT1; ++it) {
+        const int r = it * NT + ((tid - CW - W0) & (NT - 1)), o = 1 + IT0 + it;
+        slot[o] = -1;
+        if (r < h1) {
+            int x, y, z;
+            split3(r, n0, 2 * G, x, y, z);
+            slot[o] = C::B1 + x + TX * (y + 2 * G * z);
+            const CellSrc src = cell_source<DIM, 1>(ctx, tlo[0] + x, tlo[1] + (y < G ? y - G : n1 + y - G), tlo[2] + z, bad);
+            load_cell<DIM, NP>(src, Uc[o]);
+            flip[o] = src.flip;
+        }
+    }
+#pragma unroll
+    for (int it = 0; it < IT2; ++it) {
+        const int r = it * NT + ((tid - CW - W0 - W1) & (NT - 1)), o = 1 + IT0 + IT1 + it;
+        slot[o] = -1;
+        if (r < h2) {
+            int x, y, z;
+            split3(r, n0, n1, x, y, z);
+            slot[o] = C::B2 + x + TX * (y + TY * z);
+            const CellSrc src = cell_source<DIM, (DIM == 3 ? 2 : 1)>(ctx, tlo[0] + x, tlo[1] + y,
+                                                                     tlo[2] + (z < G ? z - G : n2 + z - G), bad);
+            load_cell<DIM, NP>(src, Uc[o]);
+            flip[o] = src.flip;
+        }
+    }
+#pragma unroll
+    for (int o = 0; o < IT; ++o) {
+        if (slot[o] >= 0) {
+            stage_cell<DIM, NP>(kp, Uc[o], flip[o], sWF + slot[o], C::CELLS, bad);
+            if constexpr (THINC) mixed |= Uc[o][IA] > kp.thinc_eps && Uc[o][IA] < 1.0 - kp.thinc_eps;
+        }
+    }
+    // THINC's gates admit only faces next to a cell with thinc_eps < alpha1 < 1 - thinc_eps: a tile without
+    // one skips them and the face normals' alpha1 (256^3 droplet: stage 3.12 -> 2.92 ms)
+    bool iface = false;
+    if constexpr (THINC) {
+        iface = __syncthreads_or(mixed);   // (the staged cells are complete)
+        if (iface) {
+            const int m0 = n0 + 2, m1 = n1 + 2, m2 = (DIM == 3) ? n2 + 2 : 1;
+            for (int r = tid; r < m0 * m1 * m2; r += NT) {
+                int x, y, z;
+                split3(r, m0, m1, x, y, z);
+                const int as = x + C::AX * (y + C::AY * z);
+                x -= 1;
+                y -= 1;
+                z -= (DIM == 3) ? 1 : 0;
+                const bool ox = x < 0 || x >= n0, oy = y < 0 || y >= n1, oz = z < 0 || z >= n2;
+                const int out = (ox ? 1 : 0) + (oy ? 1 : 0) + (oz ? 1 : 0);
+                if (out > 2) continue;   // the corners of a 3D tile: no normal reads them
+                if (out == 2) {          // one beyond the tile along two directions: not staged
+                    sA[as] = alpha_at<DIM>(ctx, tlo[0] + x, tlo[1] + y, tlo[2] + z, bad);
+                    continue;
+                }
+                int s = x + TX * (y + TY * z);
+                if (ox) s = C::B0 + (x < 0 ? G - 1 : G) + 2 * G * (y + TY * z);
+                if (oy) s = C::B1 + x + TX * ((y < 0 ? G - 1 : G) + 2 * G * z);
+                if (oz) s = C::B2 + x + TX * (y + TY * (z < 0 ? G - 1 : G));
+                sA[as] = sWF[IA * C::CELLS + s];
+            }
+        }
+    }
+    __syncthreads();
+    // (a thread's staging error is kept beside what its faces then make of such a state)
+    const int bad_state = bad;
+    bad = 0;
+
+    // 2. the faces: list index -> direction d and position (x the low face of cell x along d); only as many as
+    // the tile's real extents have, so a clipped tile leaves whole waves without work. RND a thread, the last
+    // round first: all but the first keep their fluxes in registers (Fk, Fj) until every face has read the
+    // staged primitives.
+    const int nf0 = (n0 + 1) * n1 * n2, nf01 = nf0 + n0 * (n1 + 1) * n2;
+    const int nf = nf01 + (DIM == 3 ? n0 * n1 * (n2 + 1) : 0);
+    double Fl[N], Fk[RND > 1 ? N + 1 : 1], Fj[RND > 2 ? N + 1 : 1], un = 0.0;
+#pragma unroll 1
+    for (int rd = RND - 1; rd >= 0; --rd) {
+        const int f = rd * NT + tid;
+        if (f < nf) {
+            int x, y, z;
+            const int d = (f >= nf0 ? 1 : 0) + ((DIM == 3 && f >= nf01) ? 1 : 0);
+            split3(f - (d == 0 ? 0 : (d == 1 ? nf0 : nf01)), n0 + (d == 0 ? 1 : 0), n1 + (d == 1 ? 1 : 0), x, y, z);
+            // LDS slots of the 2 G stencil cells: cell a + t - G along d is one of the tile's, or of the
+            // layers below (only for t < G) or above it (only for t >= G)
+            const int a = (d == 0) ? x : ((d == 1) ? y : z);
+            const int nd = (d == 0) ? n0 : ((d == 1) ? n1 : n2);
+            const int cs = (d == 0) ? 1 : ((d == 1) ? TX : TX * TY);
+            const int x0 = (d == 0) ? 0 : x, y0 = (d == 1) ? 0 : y, z0 = (d == 2) ? 0 : z;
+            const int core = x0 + TX * (y0 + TY * z0);
+            const int lay = (d == 0) ? C::B0 + 2 * G * (y + TY * z)
+                                     : ((d == 1) ? C::B1 + x + TX * 2 * G * z : C::B2 + x + TX * y);
+            int at[2 * G];
+#pragma unroll
+            for (int t = 0; t < 2 * G; ++t) {
+                const int c = a + t - G;
+                const int b = (t < G) ? (c < 0 ? lay + G * cs : core) : (c >= nd ? lay + (G - nd) * cs : core);
+                at[t] = b + c * cs;
+            }
+            auto st = [&](int t, int q) -> double { return sWF[q * C::CELLS + at[t]]; };
+            double c;
+            if constexpr (NP > 0) {
+                un = np_face_flux<DIM, SCHEME, RIEMANN, (NP > 0 ? NP : 2)>(kp, limiter, d, st, Fl, c, bad);
+            } else {
+                // o_d along d, o_1 and o_2 along the other directions in ascending order
+                const int s0 = (d == 0) ? 1 : ((d == 1) ? C::AX : C::AX * C::AY);
+                const int s1 = (d == 0) ? C::AX : 1, s2 = (d == 2) ? C::AX : C::AX * C::AY;
+                const int ab = (x + 1) + C::AX * ((y + 1) + C::AY * (DIM == 3 ? z + 1 : 0));
+                auto aa = [&](int od, int o1, int o2) -> double { return sA[ab + od * s0 + o1 * s1 + o2 * s2]; };
+                auto normal = [&]() -> double { return face_normal_component<DIM>(kp, d, aa); };
+                double aL = -1.0, aR = -1.0;
+                if constexpr (THINC) {
+                    if (iface) thinc_decide<DIM, G>(kp, st, normal, aL, aR);
+                }
+                un = face_flux_decided<DIM, SCHEME, RIEMANN, THINC>(kp, limiter, d, st, aL, aR, Fl, c, bad);
+            }
+            // the high face of the tile's last cells belongs to the next tile (or to none)
+            if (a < nd) {
+                if (__builtin_isnan(c)) bad = CMP_ERR_NAN;
+                cmax_loc = smax(cmax_loc, c);
+            }
+        }
+        if constexpr (RND > 1) {
+            if (rd == 1) {
+#pragma unroll
+                for (int q = 0; q < N; ++q) Fk[q] = Fl[q];
+                Fk[N] = un;
+            }
+        }
+        if constexpr (RND > 2) {
+            if (rd == 2) {
+#pragma unroll
+                for (int q = 0; q < N; ++q) Fj[q] = Fl[q];
+                Fj[N] = un;
+            }
+        }
+    }
+    __syncthreads();
+    if (tid < nf) {
+#pragma unroll
+        for (int q = 0; q < N; ++q) sWF[q * C::FACES + tid] = Fl[q];
+        sWF[N * C::FACES + tid] = un;
+    }
+    if constexpr (RND > 1) {
+        if (NT + tid < nf) {
+#pragma unroll
+            for (int q = 0; q <= N; ++q) sWF[q * C::FACES + NT + tid] = Fk[q];
+        }
+    }
+    if constexpr (RND > 2) {
+        if (2 * NT + tid < nf) {
+#pragma unroll
+            for (int q = 0; q <= N; ++q) sWF[q * C::FACES + 2 * NT + tid] = Fj[q];
+        }
+    }
+    __syncthreads();
+    // 3. flux differences of the thread's cell, and its update
+    if (valid) {
+        double acc[N], divu = 0.0;
+#pragma unroll
+        for (int d = 0; d < DIM; ++d) {
+            const int fm = (d == 0) ? cx + (n0 + 1) * (cy + n1 * cz)
+                         : ((d == 1) ? nf0 + cx + n0 * (cy + (n1 + 1) * cz) : nf01 + cx + n0 * (cy + n1 * cz));
+            const int fp = fm + ((d == 0) ? 1 : ((d == 1) ? n0 : n0 * n1));
+            const double idx = kp.inv_dx[d];
+#pragma unroll
+            for (int q = 0; q < N; ++q) {
+                const double v = (sWF[q * C::FACES + fp] - sWF[q * C::FACES + fm]) * idx;
+                acc[q] = (d == 0) ? v : acc[q] + v;
+            }
+            const double v = (sWF[N * C::FACES + fp] - sWF[N * C::FACES + fm]) * idx;
+            divu = (d == 0) ? v : divu + v;
+        }
+        update_cell<DIM, SCHEME, RIEMANN, NP>(kp, mode, stage, bx, tlo[0] + cx, tlo[1] + cy, tlo[2] + cz, acc, divu, Ub,
+                                              Un, Uout, dtp, bad);
+    }
+    if (cmax_bits) reduce_cmax(cmax_loc, cmax_bits, sRed, tid);
+    bad = max(bad, bad_state);
+    if (bad && err) atomicMax(err, bad);
+}
+
+// Which stages go direction by direction (pass_tile): the Phase-Field flux, whose tiles mostly have no face to
+// compute and want many small workgroups (256^3 droplet: 0.44 ms a stage, 0.75 ms as a face list), and the
+// N-phase model. Its hierarchies interpolate ghost cells with one slope factor for all components, which turns
+// a state's last bits into 1e-6 of a run's difference after a few steps: it keeps the arithmetic it has, bit
+// for bit (as a face list, in weno5_pair's form, five steps of 512^2 took 0.54 ms against 0.91).
+template <int RIEMANN, int NP>
+struct StagePasses { static constexpr bool on = RIEMANN >= RIEMANN_PF_MIX || NP > 0; };
+
+// Minimum resident waves per SIMD the register allocator must leave room for: as many as LDS admits
+// workgroups (four waves each, one a SIMD). The flow in 3D stages 48 to 53 KB: three; in 2D 29 KB: four at 107
+// VGPRs. WENO5B's two-sided limiter wants 200 VGPRs: three waves with 112 bytes of spills measured 0.54 ms for
+// five steps of 1024 x 256, two without spills 0.62 ms. The Phase-Field stage is bound by memory and takes 91
+// VGPRs by itself.
+template <int DIM, int SCHEME, int RIEMANN, int NP>
+struct StageWaves {
+    static constexpr int W = StagePasses<RIEMANN, NP>::on ? 2 : (SCHEME == 6 || DIM == 3) ? 3 : 4;
+};
+
+template <int DIM, int SCHEME, int RIEMANN, bool THINC, int NP>
+__global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(StageWaves<DIM, SCHEME, RIEMANN, NP>::W)))
 void k_stage(KParams kp, int limiter, int mode, int stage,
              const TileDev* __restrict__ tiles, int ntiles, const BoxDev* __restrict__ boxes,
              BoxDev sbox, int sntx, int snty, int single,
@@ -641,10 +935,12 @@ void k_stage(KParams kp, int limiter, int mode, int stage,
 {
     constexpr int N = NP ? 2 * NP + DIM + 1 : 4 + DIM;
     constexpr int G = Stencil<SCHEME>::G;
-    using L = Lds<DIM, G>;
-    constexpr int TX = L::TX, TY = L::TY, TZ = L::TZ;
-    // the staged primitives of a direction and, once its faces are computed, their fluxes
-    __shared__ double sWF[lds_doubles<N, LdsOf<DIM, G, ShapeFixed<DIM>>>()];
+    // direction passes (see StagePasses) or the flow's face list
+    constexpr bool PASS = StagePasses<RIEMANN, NP>::on;
+    constexpr int TX = Tile<DIM>::X, TY = Tile<DIM>::Y, TZ = Tile<DIM>::Z;
+    // the staged primitives and, once the faces are computed, their fluxes
+    __shared__ double sWF[PASS ? lds_doubles<N, LdsOf<DIM, G, ShapeFixed<DIM>>>() : Cross<DIM, G>::template doubles<N>()];
+    __shared__ double sA[THINC ? Cross<DIM, G>::ALPHAS : 1];
     __shared__ double sRed[NT / 64];
     // a step of size zero (a level clock past its stop_time) leaves every state as it is
     if (mode == MODE_RK && *dtp == 0.0) return;
@@ -676,23 +972,25 @@ void k_stage(KParams kp, int limiter, int mode, int stage,
             }
         }
     }
-    stage_tile<DIM, SCHEME, RIEMANN, THINC, NP>(kp, limiter, mode, stage, bx, tlo, ShapeFixed<DIM>{}, halo, boxes, Us,
-                                                Un, Uout, dtp, cmax_bits, err, gq, fd, sWF, sRed);
+    if constexpr (PASS)
+        pass_tile<DIM, SCHEME, RIEMANN, THINC, NP>(kp, limiter, mode, stage, bx, tlo, ShapeFixed<DIM>{}, halo, boxes, Us,
+                                                   Un, Uout, dtp, cmax_bits, err, gq, fd, sWF, sRed);
+    else
+        flow_tile<DIM, SCHEME, RIEMANN, THINC, NP>(kp, limiter, mode, stage, bx, tlo, halo, boxes, Us, Un, Uout, dtp,
+                                                   cmax_bits, err, fd, sWF, sA, sRed);
 }
 
 // One RK stage of a batch of independent levels: every tile of every admitted case in one launch.
 // A box's case is its `pad` field; each case has its own parameters, dt, c_max, error word and
 // ghost-fill tables (the halo lookup); the cells beyond a box are read from their source boxes.
 template <int DIM, int SCHEME, int RIEMANN>
-__global__ __launch_bounds__(NT) CMP_STAGE_ATTR
+__global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(StageWaves<DIM, SCHEME, RIEMANN, 0>::W)))
 void k_stage_batch(const KParams* __restrict__ kps, int limiter, int stage, const TileDev* __restrict__ tiles,
                    int ntiles, const BoxDev* __restrict__ boxes, const double* __restrict__ Us, const double* Un,
                    double* Uout, const double* __restrict__ dts, unsigned long long* cmax_bits, int* errs,
                    const FillDev* __restrict__ fds)
 {
-    constexpr int N = 4 + DIM;
-    constexpr int G = Stencil<SCHEME>::G;
-    __shared__ double sWF[lds_doubles<N, LdsOf<DIM, G, ShapeFixed<DIM>>>()];
+    __shared__ double sWF[Cross<DIM, Stencil<SCHEME>::G>::template doubles<4 + DIM>()];
     __shared__ double sRed[NT / 64];
 
     const TileDev td = tiles[xcd_tile(blockIdx.x, ntiles)];
@@ -701,9 +999,8 @@ void k_stage_batch(const KParams* __restrict__ kps, int limiter, int stage, cons
     const int tlo[3] = {td.lo[0], td.lo[1], td.lo[2]};
     const int halo[3][2] = {{td.halo[0][0], td.halo[0][1]}, {td.halo[1][0], td.halo[1][1]},
                             {td.halo[2][0], td.halo[2][1]}};
-    stage_tile<DIM, SCHEME, RIEMANN, false, 0>(kps[cs], limiter, MODE_RK, stage, bx, tlo, ShapeFixed<DIM>{}, halo,
-                                               boxes, Us, Un, Uout, dts + cs, cmax_bits + cs, errs + cs, nullptr,
-                                               fds + cs, sWF, sRed);
+    flow_tile<DIM, SCHEME, RIEMANN, false, 0>(kps[cs], limiter, MODE_RK, stage, bx, tlo, halo, boxes, Us, Un, Uout,
+                                              dts + cs, cmax_bits + cs, errs + cs, fds + cs, sWF, nullptr, sRed);
 }
 
 #ifndef CMP_LIST_UNIT
@@ -2256,9 +2553,9 @@ void k_stage_list(const ListLevel* __restrict__ levs, const ListTile* __restrict
                 halo[d][1] = td.halo[d][1];
             }
         }
-        stage_tile<DIM, SCHEME, RIEMANN, THINC, NP>(lv.kp, limiter, mode, stage, bx, tlo, sh, halo, lv.boxes,
-                                                    call.Us[l], call.Un[l], call.Uout[l], dtp, call.cmax[l], lv.err,
-                                                    nullptr, lv.fd, sWF, sRed);
+        pass_tile<DIM, SCHEME, RIEMANN, THINC, NP>(lv.kp, limiter, mode, stage, bx, tlo, sh, halo, lv.boxes,
+                                                   call.Us[l], call.Un[l], call.Uout[l], dtp, call.cmax[l], lv.err,
+                                                   nullptr, lv.fd, sWF, sRed);
     }
     if (tid == 0) {
         __threadfence();
