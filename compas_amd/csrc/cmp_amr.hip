@@ -1078,8 +1078,8 @@ int amr_comp_solve(cmp_amr* A, double* const* out, hipStream_t s0)
             m.g = L->pg;
             m.maxcells = L->maxcells;
             m.sc = scx;
-            m.src = L->d_R;
-            m.r = L->d_Z;
+            m.r = L->d_R;
+            m.dst = L->d_Z;
             m.part = L->d_part;
             CMP_TRY(dim == 2 ? launch_mg_dim<2>(MG_CG_RZ, m, s) : launch_mg_dim<3>(MG_CG_RZ, m, s));
         }

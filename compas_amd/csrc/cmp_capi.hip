@@ -1421,52 +1421,36 @@ int cmp::mg_vcycle(cmp_level* L, const double* sc, size_t m, hipStream_t s)
 {
     const int dim = L->P.dim;
     auto& V = L->mg[m];
-    if (V.G.nc <= cmp::MG_TAIL_MAX_CELLS && L->mg.size() - m <= (size_t)cmp::MG_TAIL_MAX_LEVELS) {
+    // the LDS of a tail from grid m on: two iterates of the first grid; iterates, residual, inverse diagonal
+    // and face coefficients of every coarser one
+    cmp::MgTail t{};
+    t.nlev = (int)(L->mg.size() - m);
+    bool tail = V.G.nc <= cmp::MG_TAIL_MAX_CELLS && t.nlev <= cmp::MG_TAIL_MAX_LEVELS;
+    long long off = 0;
+    for (int q = 0; tail && q < t.nlev; ++q) {
+        t.G[q] = L->mg[m + q].G;
+        const long long nc = t.G[q].nc;
+        for (int a = 0; a < (q ? 4 : 2); ++a, off += nc) t.loff[q][a] = (int)off;
+        for (int d = 0; q && d < dim; ++d) {
+            t.loff[q][4 + d] = (int)off;
+            long long nf = 1;
+            for (int e = 0; e < dim; ++e) nf *= t.G[q].n[e] + (e == d);
+            off += nf;
+        }
+        tail = off <= cmp::MG_TAIL_LDS && (q == 0 || nc <= 1024);
+    }
+    if (tail) {
         // this grid and every coarser one in a single workgroup (one launch instead of six a grid)
-        cmp::MgTail t{};
-        t.nlev = (int)(L->mg.size() - m);
         t.sweeps = L->mg_bottom_sweeps;
         t.omega = L->mg_omega;
         t.sc = sc;
         for (int q = 0; q < t.nlev; ++q) {
             const auto& W = L->mg[m + q];
-            t.G[q] = W.G;
             t.x0[q] = W.x[0];
             t.x1[q] = W.x[1];
             t.r[q] = W.r;
             t.id[q] = W.id;
             for (int d = 0; d < 3; ++d) t.b[q][d] = W.b[d];
-        }
-        // the coarsest grids that fit the tail's LDS together (never the first, whose result the
-        // caller reads from device memory)
-        auto need = [&](int q) -> long long {
-            long long n = 4 * t.G[q].nc;
-            for (int d = 0; d < dim; ++d) {
-                long long nf = 1;
-                for (int e = 0; e < dim; ++e) nf *= t.G[q].n[e] + (e == d);
-                n += nf;
-            }
-            return n;
-        };
-        t.lds_from = t.nlev;
-        long long used = 0;
-        for (int q = t.nlev - 1; q >= 1 && used + need(q) <= cmp::MG_TAIL_LDS; --q) {
-            used += need(q);
-            t.lds_from = q;
-        }
-        long long off = 0;
-        for (int q = t.lds_from; q < t.nlev; ++q) {
-            const long long nc = t.G[q].nc;
-            for (int a = 0; a < 4; ++a) t.loff[q][a] = (int)(off + a * nc);
-            off += 4 * nc;
-            for (int d = 0; d < 3; ++d) {
-                t.loff[q][4 + d] = (int)off;
-                if (d < dim) {
-                    long long nf = 1;
-                    for (int e = 0; e < dim; ++e) nf *= t.G[q].n[e] + (e == d);
-                    off += nf;
-                }
-            }
         }
         CMP_TRY(dim == 2 ? cmp::launch_mg_tail_dim<2>(t, s) : cmp::launch_mg_tail_dim<3>(t, s));
         V.cur = (t.nlev == 1) ? 0 : 1;
@@ -1484,11 +1468,7 @@ int cmp::mg_vcycle(cmp_level* L, const double* sc, size_t m, hipStream_t s)
         V.cur = 0;
         return mg_launch(dim, cmp::MG_BOTTOM, a, s);
     }
-    a.zero_x = 1;
-    a.dst = V.x[0];
-    if ((r = mg_launch(dim, cmp::MG_SMOOTH, a, s))) return r;
-    a.zero_x = 0;
-    a.src = V.x[0];
+    a.from = cmp::MG_FROM_ZERO;
     a.dst = V.x[1];
     if ((r = mg_launch(dim, cmp::MG_SMOOTH, a, s))) return r;
     auto& C = L->mg[m + 1];
@@ -1497,12 +1477,11 @@ int cmp::mg_vcycle(cmp_level* L, const double* sc, size_t m, hipStream_t s)
     a.Gc = C.G;
     if ((r = mg_launch(dim, cmp::MG_RESID_RESTRICT, a, s))) return r;
     if ((r = mg_vcycle(L, sc, m + 1, s))) return r;
-    a.src = C.x[C.cur];
-    a.dst = V.x[1];
-    if ((r = mg_launch(dim, cmp::MG_PROLONG, a, s))) return r;
-    a.src = V.x[1];
+    a.from = cmp::MG_FROM_COARSE;
+    a.xc = C.x[C.cur];
     a.dst = V.x[0];
     if ((r = mg_launch(dim, cmp::MG_SMOOTH, a, s))) return r;
+    a.from = cmp::MG_FROM_X;
     a.src = V.x[0];
     a.dst = V.x[1];
     if ((r = mg_launch(dim, cmp::MG_SMOOTH, a, s))) return r;
@@ -1524,9 +1503,7 @@ static int mg_precondition(cmp_level* L, const double* sc, hipStream_t s)
     if (r) return r;
     a.src = L->mg[0].x[L->mg[0].cur];
     a.dst = L->d_Z;
-    if ((r = mg_launch(dim, cmp::MG_SCATTER, a, s))) return r;
-    a.src = L->d_R;
-    a.r = L->d_Z;
+    a.r = L->d_R;
     a.part = L->d_part;
     return mg_launch(dim, cmp::MG_CG_RZ, a, s);
 }
@@ -1563,10 +1540,9 @@ static int pf_gradq_implicit(cmp_level* L, double dt, double eta, double* gradq,
         if (!r) r = mg_precondition(L, nullptr, s);
         if (r) return r;
     }
-    CMP_TRY(launch_reduce_sums(L->d_part, L->nblocks, 2, sc + CG_RR, s));
+    CMP_TRY(launch_reduce_sums(L->d_part, L->nblocks, mg ? 4 : 2, sc + CG_RR, s, nullptr, sc + CG_ZS));
     if (mg) {
         // p = z - mean(z)
-        CMP_TRY(launch_reduce_sums(L->d_part + 2 * (long long)L->nblocks, L->nblocks, 2, sc + CG_ZS, s));
         CMP_TRY(launch_cg_start(sc, s, inv_n));
         CMP_TRY(launch_cg_p(dim, L->pg, L->maxcells, sc, L->d_Z, L->d_Pv, s, inv_n, nullptr, 1));
     } else {
@@ -1587,10 +1563,7 @@ static int pf_gradq_implicit(cmp_level* L, double dt, double eta, double* gradq,
                 int r = mg_precondition(L, sc, cs);
                 if (r) return r;
             }
-            CMP_TRY(launch_reduce_sums(L->d_part, L->nblocks, 2, sc + CG_RRNEW, cs, sc));
-            if (mg)
-                CMP_TRY(launch_reduce_sums(L->d_part + 2 * (long long)L->nblocks, L->nblocks, 2, sc + CG_ZS, cs,
-                                           sc));
+            CMP_TRY(launch_reduce_sums(L->d_part, L->nblocks, mg ? 4 : 2, sc + CG_RRNEW, cs, sc, sc + CG_ZS));
             CMP_TRY(launch_cg_p(dim, L->pg, L->maxcells, sc, L->d_Z, L->d_Pv, cs, inv_n));
             CMP_TRY(launch_cg_end(sc, maxit, cs, inv_n));
         }

@@ -318,17 +318,17 @@ struct MgGrid {
 };
 
 enum MgOp {
-    MG_GATHER_R, MG_SCATTER, MG_GATHER_B, MG_RESTRICT_B, MG_DIAG, MG_SMOOTH, MG_RESID_RESTRICT, MG_PROLONG,
-    MG_BOTTOM, MG_CG_RZ
+    MG_GATHER_R, MG_GATHER_B, MG_RESTRICT_B, MG_DIAG, MG_SMOOTH, MG_RESID_RESTRICT, MG_BOTTOM, MG_CG_RZ
 };
 
 // Arguments of one multigrid operation (the fields an operation does not use are ignored):
-//   GATHER_R: src (box layout) -> dst (dense G); SCATTER: src (dense G) -> dst (box layout);
-//   GATHER_B: src (box face buffer) -> b[d] (dense faces); RESTRICT_B: b[d] (G) -> bc[d] (Gc);
-//   DIAG: b -> dst = 1/diag; SMOOTH: dst = src + omega id (r - A src) (zero_x: src = 0);
-//   RESID_RESTRICT: dst (Gc) = mean of the children of r - A src (G); PROLONG: dst (G) += src (Gc);
-//   BOTTOM: dst = `sweeps` Jacobi sweeps from 0 on r (G at most 1024 cells);
-//   CG_RZ: r.z partials of src (R) and r (Z) into part's second slot, dst (P) = Z when non-null.
+//   GATHER_R: src (box layout) -> dst (dense G); GATHER_B: src (box face buffer) -> b[d] (dense faces);
+//   RESTRICT_B: b[d] (G) -> bc[d] (Gc); DIAG: b -> dst = 1/diag; SMOOTH: dst = x + omega id (r - A x),
+//   x as `from` says (src, zero swept once, src plus xc on Gc); RESID_RESTRICT: dst (Gc) = mean of the
+//   children of r - A src (G); BOTTOM: dst = `sweeps` Jacobi sweeps from 0 on r (G at most 1024 cells);
+//   CG_RZ: partials of r.z, z and r into part's second to fourth slots, r and dst (= z) in box layout; z
+//   taken from src (dense G) into dst first when src is non-null.
+enum MgFrom { MG_FROM_X = 0, MG_FROM_ZERO = 1, MG_FROM_COARSE = 2 };
 struct MgArgs {
     PfGeom g;
     long long maxcells;
@@ -342,8 +342,9 @@ struct MgArgs {
     double* bc[3];
     double* part;
     MgGrid G, Gc;
+    const double* xc;
     double omega;
-    int zero_x;
+    int from;
     int sweeps;
 };
 
@@ -354,12 +355,12 @@ hipError_t launch_mg_dim(int op, const MgArgs& a, hipStream_t s);
 // the residual of grid 0 ready in r[0]; the same operations in the same order as the per-grid
 // launches (two damped Jacobi sweeps, residual restriction, the coarser grids, prolongation, two
 // sweeps; the last grid `sweeps` sweeps from zero), the result in x1[0] (x0[0] when nlev is 1).
-// Grids lds_from..nlev-1 (lds_from >= 1) live in the workgroup's LDS for the whole tail (their
-// iterates, residual, inverse diagonal and face coefficients at the double offsets loff[m][0..6]:
-// x0, x1, r, id, b0, b1, b2; id and b copied in first), the others in device memory.
+// The iterates of every grid and the residual, inverse diagonal and face coefficients of all but the
+// first live in the workgroup's LDS, at the double offsets loff[m][0..6]: x0, x1, r, id, b0, b1, b2 (the
+// first grid: x0, x1 alone). Every grid but the first has at most 1024 cells (one a thread).
 constexpr int MG_TAIL_MAX_LEVELS = 16;
 constexpr long long MG_TAIL_MAX_CELLS = 4096;   // grids at most this size go to the tail
-constexpr int MG_TAIL_LDS = 9216;               // doubles of LDS for the tail's coarsest grids
+constexpr int MG_TAIL_LDS = 17408;              // doubles of LDS: 4096 cells and what lies below them
 struct MgTail {
     int nlev;
     int sweeps;
@@ -371,7 +372,6 @@ struct MgTail {
     double* r[MG_TAIL_MAX_LEVELS];
     const double* id[MG_TAIL_MAX_LEVELS];
     const double* b[MG_TAIL_MAX_LEVELS][3];
-    int lds_from;
     int loff[MG_TAIL_MAX_LEVELS][7];
 };
 template <int DIM>
@@ -547,10 +547,10 @@ hipError_t launch_cg_end(double* sc, int maxit, hipStream_t s, double inv_n = 0.
 // face gradient of x (ghosts filled), zero on Neumann domain faces, with max |.|
 hipError_t launch_pf_gradx(int dim, const PfGeom& g, const long long* maxfaces, const double* X,
                            double* gq, unsigned long long* gmax_bits, int* boxflag, hipStream_t s);
-// sums[v] = the sum of the nblocks partials of value v (fixed order); sc non-null: nothing once the
-// CG's stop flag sc[CG_DONE] is set
+// sums[v] = the sum of the nblocks partials of value v (fixed order), values 2 and 3 into sums2[0] and
+// sums2[1]; sc non-null: nothing once the CG's stop flag sc[CG_DONE] is set
 hipError_t launch_reduce_sums(const double* part, int nblocks, int nvals, double* sums, hipStream_t s,
-                              const double* sc = nullptr);
+                              const double* sc = nullptr, double* sums2 = nullptr);
 // The partial sums of every level of a composite solve in one launch: per level the same fixed-order
 // reduction as launch_reduce_sums (into per[l * nvals + v]), then sums[v] = the levels' values added
 // in level order.

@@ -49,14 +49,12 @@ __device__ __forceinline__ long long mg_face(const MgGrid& G, int d, int i, int 
 }
 
 // (A x)_c = -div(b grad x) at cell (i,j,k): sum_d (b_lo (x_c - x_m) - b_hi (x_p - x_c)) / h_d^2, with
-// no flux through a Neumann domain face and periodic neighbours wrapped
-template <int DIM>
-__device__ __forceinline__ double mg_apply(const MgGrid& G, const double* __restrict__ x, const double* const* b,
-                                           int i, int j, int k)
+// no flux through a Neumann domain face and periodic neighbours wrapped; x(i,j,k) the value at a cell
+template <int DIM, typename X>
+__device__ __forceinline__ double mg_apply(const MgGrid& G, const X& x, const double* const* b, int i, int j, int k)
 {
     const int co[3] = {i, j, k};
-    const long long c = mg_idx(G, i, j, k);
-    const double xc = x[c];
+    const double xc = x(i, j, k);
     double acc = 0.0;
 #pragma unroll
     for (int d = 0; d < DIM; ++d) {
@@ -65,16 +63,23 @@ __device__ __forceinline__ double mg_apply(const MgGrid& G, const double* __rest
         m[d] = lo_dom ? G.n[d] - 1 : co[d] - 1;
         p[d] = hi_dom ? 0 : co[d] + 1;
         double flo = 0.0, fhi = 0.0;
-        if (!lo_dom || G.periodic[d]) flo = b[d][mg_face(G, d, i, j, k)] * (xc - x[mg_idx(G, m[0], m[1], m[2])]);
+        if (!lo_dom || G.periodic[d]) flo = b[d][mg_face(G, d, i, j, k)] * (xc - x(m[0], m[1], m[2]));
         if (!hi_dom || G.periodic[d]) {
             int f[3] = {i, j, k};
             f[d] += 1;
-            fhi = b[d][mg_face(G, d, f[0], f[1], f[2])] * (x[mg_idx(G, p[0], p[1], p[2])] - xc);
+            fhi = b[d][mg_face(G, d, f[0], f[1], f[2])] * (x(p[0], p[1], p[2]) - xc);
         }
         acc += (flo - fhi) * G.ih2[d];
     }
     return acc;
 }
+
+// the values of a grid's array
+struct MgValues {
+    const MgGrid& G;
+    const double* x;
+    __device__ __forceinline__ double operator()(int i, int j, int k) const { return x[mg_idx(G, i, j, k)]; }
+};
 
 template <int DIM>
 __global__ __launch_bounds__(NT) void k_mg_gather_r(PfGeom g, const double* __restrict__ sc,
@@ -92,24 +97,6 @@ __global__ __launch_bounds__(NT) void k_mg_gather_r(PfGeom g, const double* __re
     j += ab.lo[1];
     k += ab.lo[2];
     r0[mg_idx(G, i - g.dlo[0], j - g.dlo[1], (DIM == 3) ? k - g.dlo[2] : 0)] = R[ab.off + fab_index(ab, i, j, k)];
-}
-
-template <int DIM>
-__global__ __launch_bounds__(NT) void k_mg_scatter(PfGeom g, const double* __restrict__ sc,
-                                                   const double* __restrict__ x0, double* Z, MgGrid G)
-{
-    if (sc && sc[CG_DONE] != 0.0) return;
-    long long q;
-    const BoxDev ab = g.abox[cell_block(g.cmap, q)];
-    const int n0 = ab.hi[0] - ab.lo[0] + 1, n1 = ab.hi[1] - ab.lo[1] + 1;
-    const int n2 = (DIM == 3) ? ab.hi[2] - ab.lo[2] + 1 : 1;
-    if (q >= (long long)n0 * n1 * n2) return;
-    int i, j, k;
-    pos3(q, n0, n1, i, j, k);
-    i += ab.lo[0];
-    j += ab.lo[1];
-    k += ab.lo[2];
-    Z[ab.off + fab_index(ab, i, j, k)] = x0[mg_idx(G, i - g.dlo[0], j - g.dlo[1], (DIM == 3) ? k - g.dlo[2] : 0)];
 }
 
 // the box face buffer of direction D (cmp_face_layout, one component) -> the dense face array
@@ -178,24 +165,33 @@ __global__ __launch_bounds__(NT) void k_mg_diag(const double* __restrict__ b0, c
     }
 }
 
-// one damped Jacobi sweep y = x + omega D^-1 (r - A x); zero_x: x = 0 (y = omega D^-1 r)
-template <int DIM>
+// one damped Jacobi sweep y = x + omega D^-1 (r - A x). FROM: x the array (MG_FROM_X), the sweep from zero
+// omega D^-1 r (MG_FROM_ZERO) or the array plus the coarser grid's value at the parent cell
+// (MG_FROM_COARSE), the last two computed where they are read: a launch and a pass over memory each against
+// one or two more loads a neighbour, all from cache: four launches a
+// grid instead of six. With one launch for z's scatter and the sums and one for four sums, a 512 x 256 Grad_Q
+// 2.68 -> 2.31 ms, eight cases' CAC steps 7.90 -> 6.92 ms.
+template <int DIM, int FROM>
 __global__ __launch_bounds__(NT) void k_mg_smooth(const double* __restrict__ sc, const double* __restrict__ x,
                                                   double* __restrict__ y, const double* __restrict__ r,
                                                   const double* __restrict__ b0, const double* __restrict__ b1,
                                                   const double* __restrict__ b2, const double* __restrict__ id,
-                                                  MgGrid G, double omega, int zero_x)
+                                                  MgGrid G, double omega, const double* __restrict__ xc, MgGrid Gc)
 {
     if (sc && sc[CG_DONE] != 0.0) return;
     const double* b[3] = {b0, b1, b2};
+    auto value = [&](int i, int j, int k) __attribute__((always_inline)) -> double {
+        // (rounded as a value that was stored: no term of it is contracted into a difference)
+#pragma clang fp contract(off)
+        const long long c = mg_idx(G, i, j, k);
+        if (FROM == MG_FROM_ZERO) return omega * id[c] * r[c];
+        if (FROM == MG_FROM_COARSE) return x[c] + xc[mg_idx(Gc, i >> 1, j >> 1, (DIM == 3) ? (k >> 1) : 0)];
+        return x[c];
+    };
     for (long long q = (long long)blockIdx.x * NT + threadIdx.x; q < G.nc; q += (long long)gridDim.x * NT) {
-        if (zero_x) {
-            y[q] = omega * id[q] * r[q];
-        } else {
-            int i, j, k;
-            mg_cell<DIM>(G, q, i, j, k);
-            y[q] = x[q] + omega * id[q] * (r[q] - mg_apply<DIM>(G, x, b, i, j, k));
-        }
+        int i, j, k;
+        mg_cell<DIM>(G, q, i, j, k);
+        y[q] = value(i, j, k) + omega * id[q] * (r[q] - mg_apply<DIM>(G, value, b, i, j, k));
     }
 }
 
@@ -217,22 +213,9 @@ __global__ __launch_bounds__(NT) void k_mg_resid_restrict(const double* __restri
         for (int ch = 0; ch < NCH; ++ch) {
             const int i = 2 * I + (ch & 1), j = 2 * J + ((ch >> 1) & 1), k = (DIM == 3) ? 2 * K + (ch >> 2) : 0;
             const long long c = mg_idx(Gf, i, j, k);
-            s += r[c] - mg_apply<DIM>(Gf, x, b, i, j, k);
+            s += r[c] - mg_apply<DIM>(Gf, MgValues{Gf, x}, b, i, j, k);
         }
         rc[q] = s * (1.0 / (double)NCH);
-    }
-}
-
-// x_fine += x_coarse of the parent cell
-template <int DIM>
-__global__ __launch_bounds__(NT) void k_mg_prolong(const double* __restrict__ sc, const double* __restrict__ xc,
-                                                   double* xf, MgGrid Gf, MgGrid Gc)
-{
-    if (sc && sc[CG_DONE] != 0.0) return;
-    for (long long q = (long long)blockIdx.x * NT + threadIdx.x; q < Gf.nc; q += (long long)gridDim.x * NT) {
-        int i, j, k;
-        mg_cell<DIM>(Gf, q, i, j, k);
-        xf[q] += xc[mg_idx(Gc, i >> 1, j >> 1, (DIM == 3) ? (k >> 1) : 0)];
     }
 }
 
@@ -260,126 +243,285 @@ __global__ __launch_bounds__(1024) void k_mg_bottom(const double* __restrict__ s
     __syncthreads();
     int cur = 0;
     for (int s = 1; s < sweeps; ++s) {
-        if (on) xs[1 - cur][q] = xs[cur][q] + omega * iq * (rq - mg_apply<DIM>(G, xs[cur], b, i, j, k));
+        if (on) xs[1 - cur][q] = xs[cur][q] + omega * iq * (rq - mg_apply<DIM>(G, MgValues{G, xs[cur]}, b, i, j, k));
         __syncthreads();
         cur = 1 - cur;
     }
     if (on) x[q] = xs[cur][q];
 }
 
-// The coarse end of the V-cycle (MgTail) in one workgroup of 1024 threads, every operation a
-// strided loop over the grid's cells followed by a barrier. The coarsest grids (from t.lds_from on)
-// are kept in LDS, so that their many short phases wait on LDS rather than on device memory; the
-// arithmetic is the same wherever a grid lives.
+// A cell of a grid with the coefficients its operator row reads, kept in registers over the phases of a
+// visit: (A x)_c = sum_d (b_lo (x_c - x_m) - b_hi (x_p - x_c)) / h_d^2, a Neumann domain face with b = 0.
+template <int DIM>
+struct TailCell {
+    int q;                  // -1: no cell
+    unsigned edge;          // bit 2d / 2d + 1: at the low / high side of the domain along d
+    double r, id, bl[DIM], bh[DIM];
+};
+
+template <int DIM>
+__device__ __forceinline__ void tail_pos(const MgGrid& G, int q, int* c)
+{
+    // exact below 10^6: the quotient (q + 1/2) / n lies at least 1/(2 n) from an integer
+    const float h = (float)q + 0.5f;
+    const int a = (int)(h * __builtin_amdgcn_rcpf((float)G.n[0]));
+    c[0] = q - a * G.n[0];
+    c[1] = a;
+    c[2] = 0;
+    if (DIM == 3) {
+        c[2] = (int)(h * __builtin_amdgcn_rcpf((float)(G.n[0] * G.n[1])));
+        c[1] = a - c[2] * G.n[1];
+    }
+}
+
+// b[d]: the grid's face coefficients
+template <int DIM, typename B>
+__device__ __forceinline__ TailCell<DIM> tail_cell(const MgGrid& G, int q, double r, double id, const B& b)
+{
+    TailCell<DIM> c;
+    int p[3];
+    tail_pos<DIM>(G, q, p);
+    c.q = q;
+    c.edge = 0u;
+    c.r = r;
+    c.id = id;
+#pragma unroll
+    for (int d = 0; d < DIM; ++d) {
+        const bool lo = p[d] == 0, hi = p[d] == G.n[d] - 1;
+        c.edge |= (lo ? 1u : 0u) << (2 * d) | (hi ? 2u : 0u) << (2 * d);
+        int f[3] = {p[0], p[1], p[2]};
+        c.bl[d] = (!lo || G.periodic[d]) ? b(d, (int)mg_face(G, d, f[0], f[1], f[2])) : 0.0;
+        f[d] += 1;
+        c.bh[d] = (!hi || G.periodic[d]) ? b(d, (int)mg_face(G, d, f[0], f[1], f[2])) : 0.0;
+    }
+    return c;
+}
+
+template <int DIM>
+__device__ __forceinline__ double tail_apply(const MgGrid& G, const TailCell<DIM>& c, const double* x)
+{
+    const double xc = x[c.q];
+    double acc = 0.0;
+#pragma unroll
+    for (int d = 0; d < DIM; ++d) {
+        const int s = (d == 0) ? 1 : ((d == 1) ? G.n[0] : G.n[0] * G.n[1]);
+        const int wrap = (G.n[d] - 1) * s;   // (a Neumann side's neighbour counts nothing: b = 0)
+        const int m = (c.edge >> (2 * d) & 1u) ? c.q + wrap : c.q - s;
+        const int p = (c.edge >> (2 * d) & 2u) ? c.q - wrap : c.q + s;
+        acc += (c.bl[d] * (xc - x[m]) - c.bh[d] * (x[p] - xc)) * G.ih2[d];
+    }
+    return acc;
+}
+
+// The coarse end of the V-cycle (MgTail) in one workgroup of 1024 threads. Bound by the latency of its many
+// short phases, so: every grid's iterates live in LDS (the first grid's r, 1/diag and b in its threads'
+// registers, at most four cells a thread; the others' in LDS), and the grids of at most 64 cells are one
+// wave's, whose phases follow each other without a barrier (its LDS accesses execute in order). The arithmetic
+// is the per-grid launches'. On one card 33 -> 14.5 us a
+// visit from 64 x 32 cells, 70 -> 24.9 from 128 x 32.
 constexpr int NTAIL = 1024;
 template <int DIM>
 __global__ __launch_bounds__(NTAIL) void k_mg_tail(MgTail t)
 {
     if (t.sc && t.sc[CG_DONE] != 0.0) return;
     __shared__ double lds[MG_TAIL_LDS];
+    constexpr int CPT = (int)(MG_TAIL_MAX_CELLS / NTAIL);
+    constexpr int NCH = (DIM == 3) ? 8 : 4;
     const int tid = threadIdx.x;
     const double om = t.omega;
     const int last = t.nlev - 1;
-    auto in_lds = [&](int m) { return m >= t.lds_from; };
-    auto X0 = [&](int m) -> double* { return in_lds(m) ? lds + t.loff[m][0] : t.x0[m]; };
-    auto X1 = [&](int m) -> double* { return in_lds(m) ? lds + t.loff[m][1] : t.x1[m]; };
-    auto Rr = [&](int m) -> double* { return in_lds(m) ? lds + t.loff[m][2] : t.r[m]; };
-    auto ID = [&](int m) -> const double* { return in_lds(m) ? lds + t.loff[m][3] : t.id[m]; };
-    auto Bf = [&](int m, int d) -> const double* { return in_lds(m) ? lds + t.loff[m][4 + d] : t.b[m][d]; };
-    // the LDS grids' inverse diagonals and face coefficients
-    for (int m = t.lds_from; m < t.nlev; ++m) {
+    int w = 1;                      // the first grid (after grid 0) that one wave takes
+    while (w <= last && t.G[w].nc > 64) ++w;
+    // the coarser grids' inverse diagonals and face coefficients
+    for (int m = 1; m < t.nlev; ++m) {
         const MgGrid& G = t.G[m];
-        for (long long q = tid; q < G.nc; q += NTAIL) lds[t.loff[m][3] + q] = t.id[m][q];
+        for (int q = tid; q < (int)G.nc; q += NTAIL) lds[t.loff[m][3] + q] = t.id[m][q];
+#pragma unroll
         for (int d = 0; d < DIM; ++d) {
-            long long nf = 1;
+            int nf = 1;
+#pragma unroll
             for (int e = 0; e < DIM; ++e) nf *= G.n[e] + (e == d);
-            for (long long q = tid; q < nf; q += NTAIL) lds[t.loff[m][4 + d] + q] = t.b[m][d][q];
+            for (int q = tid; q < nf; q += NTAIL) lds[t.loff[m][4 + d] + q] = t.b[m][d][q];
+        }
+    }
+    // grid 0's cells
+    const MgGrid& G0 = t.G[0];
+    double* const a0 = lds + t.loff[0][0];
+    double* const a1 = lds + t.loff[0][1];
+    TailCell<DIM> c0[CPT];
+#pragma unroll
+    for (int c = 0; c < CPT; ++c) {
+        const int q = c * NTAIL + tid;
+        c0[c].q = -1;
+        if (q < (int)G0.nc)
+            c0[c] = tail_cell<DIM>(G0, q, t.r[0][q], t.id[0][q], [&](int d, int f) { return t.b[0][d][f]; });
+    }
+    auto lds_cell = [&](int m, int q) __attribute__((always_inline)) {
+        return tail_cell<DIM>(t.G[m], q, lds[t.loff[m][2] + q], lds[t.loff[m][3] + q],
+                              [&](int d, int f) { return lds[t.loff[m][4 + d] + f]; });
+    };
+    // r of grid m + 1 from the residual of grid m (in its x0), the mean over the children
+    auto restrict_to = [&](int m, int q) __attribute__((always_inline)) {
+        const MgGrid& Gf = t.G[m];
+        const double* res = lds + t.loff[m][0];
+        int p[3];
+        tail_pos<DIM>(t.G[m + 1], q, p);
+        double sum = 0.0;
+#pragma unroll
+        for (int ch = 0; ch < NCH; ++ch)
+            sum += res[(2 * p[0] + (ch & 1)) +
+                       Gf.n[0] * ((2 * p[1] + ((ch >> 1) & 1)) + Gf.n[1] * ((DIM == 3) ? 2 * p[2] + (ch >> 2) : 0))];
+        lds[t.loff[m + 1][2] + q] = sum * (1.0 / (double)NCH);
+    };
+    // grid m's x1 plus the coarser grid's result at the parent cell
+    auto prolonged = [&](int m, int q) __attribute__((always_inline)) -> double {
+        int p[3];
+        tail_pos<DIM>(t.G[m], q, p);
+        const MgGrid& Gc = t.G[m + 1];
+        const double* xc = lds + t.loff[m + 1][(m + 1 == last) ? 0 : 1];
+        return lds[t.loff[m][1] + q] + xc[(p[0] >> 1) + Gc.n[0] * ((p[1] >> 1) + Gc.n[1] * ((DIM == 3) ? p[2] >> 1 : 0))];
+    };
+    // one grid of at most n threads' cells (q = the thread's, when below nc): two sweeps from zero and the
+    // residual; prolongation and two sweeps; the coarsest grid's sweeps
+    auto down = [&](int m, int q, auto sync) __attribute__((always_inline)) {
+        const MgGrid& G = t.G[m];
+        double* x0 = lds + t.loff[m][0];
+        double* x1 = lds + t.loff[m][1];
+        const bool on = q < (int)G.nc;
+        TailCell<DIM> c;
+        c.q = -1;
+        double v = 0.0;
+        if (on) {
+            c = lds_cell(m, q);
+            v = om * c.id * c.r;
+            x0[q] = v;
+        }
+        sync();
+        if (on) x1[q] = v + om * c.id * (c.r - tail_apply<DIM>(G, c, x0));
+        sync();
+        if (on) x0[q] = c.r - tail_apply<DIM>(G, c, x1);
+        sync();
+        if (q < (int)t.G[m + 1].nc) restrict_to(m, q);
+        sync();
+    };
+    auto up = [&](int m, int q, auto sync) __attribute__((always_inline)) {
+        const MgGrid& G = t.G[m];
+        double* x0 = lds + t.loff[m][0];
+        double* x1 = lds + t.loff[m][1];
+        const bool on = q < (int)G.nc;
+        TailCell<DIM> c;
+        c.q = -1;
+        double v = 0.0;
+        if (on) {
+            c = lds_cell(m, q);
+            v = prolonged(m, q);
+            x1[q] = v;
+        }
+        sync();
+        if (on) {
+            v = v + om * c.id * (c.r - tail_apply<DIM>(G, c, x1));
+            x0[q] = v;
+        }
+        sync();
+        if (on) x1[q] = v + om * c.id * (c.r - tail_apply<DIM>(G, c, x0));
+        sync();
+    };
+    auto bottom = [&](int q, auto sync) __attribute__((always_inline)) {
+        const MgGrid& G = t.G[last];
+        double* x0 = lds + t.loff[last][0];
+        double* x1 = lds + t.loff[last][1];
+        const bool on = q < (int)G.nc;
+        TailCell<DIM> c;
+        c.q = -1;
+        double v = 0.0;
+        if (on) {
+            c = lds_cell(last, q);
+            v = om * c.id * c.r;
+        }
+        for (int sw = 1; sw < t.sweeps; ++sw) {
+            double* x = (sw & 1) ? x0 : x1;
+            if (on) x[q] = v;
+            sync();
+            if (on) v = v + om * c.id * (c.r - tail_apply<DIM>(G, c, x));
+        }
+        sync();
+        if (on) x0[q] = v;
+        sync();
+    };
+    auto block_sync = [&]() { __syncthreads(); };
+    auto wave_sync = [&]() {
+        __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+    };
+    if (last == 0) {
+        // one grid: its sweeps from zero (nc <= 1024), r in place of a coarser grid's
+        __syncthreads();
+        double v = 0.0;
+        if (c0[0].q >= 0) v = om * c0[0].id * c0[0].r;
+        for (int sw = 1; sw < t.sweeps; ++sw) {
+            double* x = (sw & 1) ? a0 : a1;
+            if (c0[0].q >= 0) x[c0[0].q] = v;
+            __syncthreads();
+            if (c0[0].q >= 0) v = v + om * c0[0].id * (c0[0].r - tail_apply<DIM>(G0, c0[0], x));
+        }
+        if (c0[0].q >= 0) t.x0[0][c0[0].q] = v;
+        return;
+    }
+    double v0[CPT];
+#pragma unroll
+    for (int c = 0; c < CPT; ++c) {
+        v0[c] = 0.0;
+        if (c0[c].q >= 0) {
+            v0[c] = om * c0[c].id * c0[c].r;
+            a0[c0[c].q] = v0[c];
         }
     }
     __syncthreads();
-    // y = x + omega id (r - A x) on grid m (zero_x: y = omega id r)
-    auto smooth = [&](int m, const double* x, double* y, bool zero_x) {
-        const MgGrid& G = t.G[m];
-        const double* r = Rr(m);
-        const double* id = ID(m);
-        const double* bb[3] = {Bf(m, 0), Bf(m, 1), Bf(m, DIM == 3 ? 2 : 1)};
-        for (long long q = tid; q < G.nc; q += NTAIL) {
-            if (zero_x) {
-                y[q] = om * id[q] * r[q];
-            } else {
-                int i, j, k;
-                mg_cell<DIM>(G, q, i, j, k);
-                y[q] = x[q] + om * id[q] * (r[q] - mg_apply<DIM>(G, x, bb, i, j, k));
-            }
-        }
-        __syncthreads();
-    };
-    for (int m = 0; m < last; ++m) {
-        smooth(m, nullptr, X0(m), true);
-        smooth(m, X0(m), X1(m), false);
-        // r of grid m + 1: the mean of the children of r - A x1
-        const MgGrid& Gf = t.G[m];
-        const MgGrid& Gc = t.G[m + 1];
-        const double* rf = Rr(m);
-        const double* x1 = X1(m);
-        const double* bb[3] = {Bf(m, 0), Bf(m, 1), Bf(m, DIM == 3 ? 2 : 1)};
-        double* rc = Rr(m + 1);
-        constexpr int NCH = (DIM == 3) ? 8 : 4;
-        for (long long q = tid; q < Gc.nc; q += NTAIL) {
-            int I, J, K;
-            mg_cell<DIM>(Gc, q, I, J, K);
-            double sum = 0.0;
 #pragma unroll
-            for (int ch = 0; ch < NCH; ++ch) {
-                const int i = 2 * I + (ch & 1), j = 2 * J + ((ch >> 1) & 1), k = (DIM == 3) ? 2 * K + (ch >> 2) : 0;
-                const long long c = mg_idx(Gf, i, j, k);
-                sum += rf[c] - mg_apply<DIM>(Gf, x1, bb, i, j, k);
-            }
-            rc[q] = sum * (1.0 / (double)NCH);
-        }
-        __syncthreads();
+    for (int c = 0; c < CPT; ++c)
+        if (c0[c].q >= 0) a1[c0[c].q] = v0[c] + om * c0[c].id * (c0[c].r - tail_apply<DIM>(G0, c0[c], a0));
+    __syncthreads();
+#pragma unroll
+    for (int c = 0; c < CPT; ++c)
+        if (c0[c].q >= 0) a0[c0[c].q] = c0[c].r - tail_apply<DIM>(G0, c0[c], a1);
+    __syncthreads();
+    if (tid < (int)t.G[1].nc) restrict_to(0, tid);
+    __syncthreads();
+    for (int m = 1; m < w && m < last; ++m) down(m, tid, block_sync);
+    if (w > last) {
+        bottom(tid, block_sync);
+    } else if (tid < 64) {
+        for (int m = w; m < last; ++m) down(m, tid, wave_sync);
+        bottom(tid, wave_sync);
+        for (int m = last - 1; m >= w; --m) up(m, tid, wave_sync);
     }
-    // the coarsest grid: `sweeps` damped Jacobi sweeps from zero, alternating x0 / x1, the result
-    // copied to x0
-    {
-        const MgGrid& G = t.G[last];
-        double* xa = X0(last);
-        double* xb = X1(last);
-        smooth(last, nullptr, xa, true);
-        for (int sw = 1; sw < t.sweeps; ++sw) {
-            smooth(last, xa, xb, false);
-            double* tmp = xa;
-            xa = xb;
-            xb = tmp;
+    __syncthreads();
+    for (int m = (w > last ? last : w) - 1; m >= 1; --m) up(m, tid, block_sync);
+#pragma unroll
+    for (int c = 0; c < CPT; ++c)
+        if (c0[c].q >= 0) v0[c] = prolonged(0, c0[c].q);
+    __syncthreads();
+#pragma unroll
+    for (int c = 0; c < CPT; ++c)
+        if (c0[c].q >= 0) a1[c0[c].q] = v0[c];
+    __syncthreads();
+#pragma unroll
+    for (int c = 0; c < CPT; ++c)
+        if (c0[c].q >= 0) {
+            v0[c] = v0[c] + om * c0[c].id * (c0[c].r - tail_apply<DIM>(G0, c0[c], a1));
+            a0[c0[c].q] = v0[c];
         }
-        if (xa != X0(last)) {
-            double* x0l = X0(last);
-            for (long long q = tid; q < G.nc; q += NTAIL) x0l[q] = xa[q];
-            __syncthreads();
-        }
-    }
-    for (int m = last - 1; m >= 0; --m) {
-        // x1 += the coarser grid's result at the parent cell, then two sweeps
-        const MgGrid& Gf = t.G[m];
-        const MgGrid& Gc = t.G[m + 1];
-        const double* xc = (m + 1 == last) ? X0(m + 1) : X1(m + 1);
-        double* x1 = X1(m);
-        for (long long q = tid; q < Gf.nc; q += NTAIL) {
-            int i, j, k;
-            mg_cell<DIM>(Gf, q, i, j, k);
-            x1[q] += xc[mg_idx(Gc, i >> 1, j >> 1, (DIM == 3) ? (k >> 1) : 0)];
-        }
-        __syncthreads();
-        smooth(m, X1(m), X0(m), false);
-        smooth(m, X0(m), X1(m), false);
-    }
+    __syncthreads();
+#pragma unroll
+    for (int c = 0; c < CPT; ++c)
+        if (c0[c].q >= 0) t.x1[0][c0[c].q] = v0[c] + om * c0[c].id * (c0[c].r - tail_apply<DIM>(G0, c0[c], a0));
 }
 
 // the partial sums of one CG iteration's r.z, sum z and sum r (the second, third and fourth partial
-// slots; the first holds r.r)
+// slots; the first holds r.r). x0 non-null: z is the dense grid's value there, written to Z on the way.
 template <int DIM>
 __global__ __launch_bounds__(NT) void k_cg_rz(PfGeom g, const double* __restrict__ sc, const double* __restrict__ R,
-                                              const double* __restrict__ Z, double* part)
+                                              const double* __restrict__ x0, double* Z, MgGrid G, double* part)
 {
     if (sc && sc[CG_DONE] != 0.0) return;
     long long q;
@@ -394,7 +536,14 @@ __global__ __launch_bounds__(NT) void k_cg_rz(PfGeom g, const double* __restrict
         j += ab.lo[1];
         k += ab.lo[2];
         const long long c = ab.off + fab_index(ab, i, j, k);
-        const double r = R[c], z = Z[c];
+        double z;
+        if (x0) {
+            z = x0[mg_idx(G, i - g.dlo[0], j - g.dlo[1], (DIM == 3) ? k - g.dlo[2] : 0)];
+            Z[c] = z;
+        } else {
+            z = Z[c];
+        }
+        const double r = R[c];
         w[0] = r * z;
         w[1] = z;
         w[2] = r;
@@ -441,10 +590,6 @@ hipError_t launch_mg_dim(int op, const MgArgs& a, hipStream_t s)
         hipLaunchKernelGGL((k_mg_gather_r<DIM>), cell_grid(a.g.cmap, a.g.ncmap, a.maxcells, a.g.nbox), dim3(NT), 0, s, a.g, a.sc, a.src,
                            a.dst, a.G);
         break;
-    case MG_SCATTER:
-        hipLaunchKernelGGL((k_mg_scatter<DIM>), cell_grid(a.g.cmap, a.g.ncmap, a.maxcells, a.g.nbox), dim3(NT), 0, s, a.g, a.sc, a.src,
-                           a.dst, a.G);
-        break;
     case MG_GATHER_B:
         hipLaunchKernelGGL((k_mg_gather_b<DIM, 0>), box_grid(a.maxfaces[0], a.g.nbox), dim3(NT), 0, s, a.g, a.src,
                            a.b[0], a.G);
@@ -464,16 +609,16 @@ hipError_t launch_mg_dim(int op, const MgArgs& a, hipStream_t s)
     case MG_DIAG:
         hipLaunchKernelGGL((k_mg_diag<DIM>), mg_grid(a.G.nc), dim3(NT), 0, s, a.b[0], a.b[1], a.b[2], a.dst, a.G);
         break;
-    case MG_SMOOTH:
-        hipLaunchKernelGGL((k_mg_smooth<DIM>), mg_grid(a.G.nc), dim3(NT), 0, s, a.sc, a.src, a.dst, a.r, a.b[0],
-                           a.b[1], a.b[2], a.id, a.G, a.omega, a.zero_x);
+    case MG_SMOOTH: {
+        const auto f = a.from == MG_FROM_X ? k_mg_smooth<DIM, MG_FROM_X>
+                       : a.from == MG_FROM_ZERO ? k_mg_smooth<DIM, MG_FROM_ZERO> : k_mg_smooth<DIM, MG_FROM_COARSE>;
+        hipLaunchKernelGGL(f, mg_grid(a.G.nc), dim3(NT), 0, s, a.sc, a.src, a.dst, a.r, a.b[0], a.b[1], a.b[2],
+                           a.id, a.G, a.omega, a.xc, a.Gc);
         break;
+    }
     case MG_RESID_RESTRICT:
         hipLaunchKernelGGL((k_mg_resid_restrict<DIM>), mg_grid(a.Gc.nc), dim3(NT), 0, s, a.sc, a.src, a.r, a.b[0],
                            a.b[1], a.b[2], a.G, a.dst, a.Gc);
-        break;
-    case MG_PROLONG:
-        hipLaunchKernelGGL((k_mg_prolong<DIM>), mg_grid(a.G.nc), dim3(NT), 0, s, a.sc, a.src, a.dst, a.G, a.Gc);
         break;
     case MG_BOTTOM:
         if (a.G.nc > 1024) return hipErrorInvalidValue;
@@ -481,8 +626,8 @@ hipError_t launch_mg_dim(int op, const MgArgs& a, hipStream_t s)
                            a.id, a.G, a.omega, a.sweeps);
         break;
     case MG_CG_RZ:
-        hipLaunchKernelGGL((k_cg_rz<DIM>), cell_grid(a.g.cmap, a.g.ncmap, a.maxcells, a.g.nbox), dim3(NT), 0, s, a.g, a.sc, a.src, a.r,
-                           a.part);
+        hipLaunchKernelGGL((k_cg_rz<DIM>), cell_grid(a.g.cmap, a.g.ncmap, a.maxcells, a.g.nbox), dim3(NT), 0, s, a.g,
+                           a.sc, a.r, a.src, a.dst, a.G, a.part);
         break;
     default:
         return hipErrorInvalidValue;

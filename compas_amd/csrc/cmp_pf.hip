@@ -771,7 +771,7 @@ hipError_t launch_zero_u64(unsigned long long* p, int n, hipStream_t s)
     return hipGetLastError();
 }
 
-// sums[v] = sum_b part[v * nblocks + b], one workgroup of 1024 threads, a fixed order of additions
+// sums[v] = sum_b part[v * nblocks + b], one workgroup of 1024 threads a sum, a fixed order of additions
 // (each thread four interleaved running sums, then the wave and workgroup sums in index order).
 // sc non-null: nothing once the solve's stop flag is set (the queued iterations past the stop).
 constexpr int NRED = 1024;
@@ -804,15 +804,15 @@ __device__ __forceinline__ double reduce_block_parts(const double* __restrict__ 
     return u;
 }
 
-__global__ __launch_bounds__(NRED) void k_reduce_sums(const double* __restrict__ part, int nblocks, int nvals,
-                                                      double* sums, const double* __restrict__ sc)
+// (the sums from the third on go to sums2)
+__global__ __launch_bounds__(NRED) void k_reduce_sums(const double* __restrict__ part, int nblocks, double* sums,
+                                                      double* sums2, const double* __restrict__ sc)
 {
     if (sc && sc[CG_DONE] != 0.0) return;
     __shared__ double red[NRED / 64];
-    for (int v = 0; v < nvals; ++v) {
-        const double u = reduce_block_parts(part + (long long)v * nblocks, nblocks, red);
-        if (threadIdx.x == 0) sums[v] = u;
-    }
+    const int v = blockIdx.x;
+    const double u = reduce_block_parts(part + (long long)v * nblocks, nblocks, red);
+    if (threadIdx.x == 0) *(v < 2 ? sums + v : sums2 + (v - 2)) = u;
 }
 
 // every level's sums (per[l * nvals + v], as k_reduce_sums leaves them) and their sum in level order
@@ -886,9 +886,10 @@ hipError_t launch_reduce_levels(const LevelParts& lp, int nvals, double* per, do
 }
 
 hipError_t launch_reduce_sums(const double* part, int nblocks, int nvals, double* sums, hipStream_t s,
-                              const double* sc)
+                              const double* sc, double* sums2)
 {
-    hipLaunchKernelGGL(k_reduce_sums, dim3(1), dim3(NRED), 0, s, part, nblocks, nvals, sums, sc);
+    if (nvals > 2 && !sums2) return hipErrorInvalidValue;
+    hipLaunchKernelGGL(k_reduce_sums, dim3(nvals), dim3(NRED), 0, s, part, nblocks, sums, sums2, sc);
     return hipGetLastError();
 }
 
