@@ -1414,10 +1414,22 @@ int cmp::mg_prepare(cmp_level* L, hipStream_t s)
     return r;
 }
 
+// the partials of r.z, z and r on grid m's z = x[cur]
+static int mg_sums(const cmp_level* L, const double* sc, size_t m, double* part, hipStream_t s)
+{
+    cmp::MgArgs a = mg_args(L, sc);
+    a.G = L->mg[m].G;
+    a.src = L->mg[m].x[L->mg[m].cur];
+    a.r = L->mg[m].r;
+    a.part = part;
+    return mg_launch(L->P.dim, cmp::MG_CG_SUMS, a, s);
+}
+
 // One V-cycle on grid m from its residual r, the result left in x[cur]: two damped Jacobi sweeps
 // (the first from zero), the residual restricted, the coarser grid's V-cycle prolonged and added,
-// two more sweeps; the coarsest grid takes its fixed number of sweeps in one workgroup.
-int cmp::mg_vcycle(cmp_level* L, const double* sc, size_t m, hipStream_t s)
+// two more sweeps; the coarsest grid takes its fixed number of sweeps in one workgroup. part non-null: the
+// partials of r.z, z and r (z the result) into part's second to fourth slots of mg_blocks values.
+int cmp::mg_vcycle(cmp_level* L, const double* sc, size_t m, hipStream_t s, double* part)
 {
     const int dim = L->P.dim;
     auto& V = L->mg[m];
@@ -1454,7 +1466,7 @@ int cmp::mg_vcycle(cmp_level* L, const double* sc, size_t m, hipStream_t s)
         }
         CMP_TRY(dim == 2 ? cmp::launch_mg_tail_dim<2>(t, s) : cmp::launch_mg_tail_dim<3>(t, s));
         V.cur = (t.nlev == 1) ? 0 : 1;
-        return CMP_OK;
+        return part ? mg_sums(L, sc, m, part, s) : CMP_OK;
     }
     cmp::MgArgs a = mg_args(L, sc);
     for (int d = 0; d < 3; ++d) a.b[d] = V.b[d];
@@ -1466,7 +1478,8 @@ int cmp::mg_vcycle(cmp_level* L, const double* sc, size_t m, hipStream_t s)
         a.dst = V.x[0];
         a.sweeps = L->mg_bottom_sweeps;
         V.cur = 0;
-        return mg_launch(dim, cmp::MG_BOTTOM, a, s);
+        if ((r = mg_launch(dim, cmp::MG_BOTTOM, a, s))) return r;
+        return part ? mg_sums(L, sc, m, part, s) : CMP_OK;
     }
     a.from = cmp::MG_FROM_ZERO;
     a.dst = V.x[1];
@@ -1484,28 +1497,64 @@ int cmp::mg_vcycle(cmp_level* L, const double* sc, size_t m, hipStream_t s)
     a.from = cmp::MG_FROM_X;
     a.src = V.x[0];
     a.dst = V.x[1];
+    a.part = part;
     if ((r = mg_launch(dim, cmp::MG_SMOOTH, a, s))) return r;
     V.cur = 1;
     return CMP_OK;
 }
 
-// z = V(r) for the CG's residual (level buffers R -> Z), then the block partials of r.z, sum z and
-// sum r into the second to fourth slots of d_part.
-static int mg_precondition(cmp_level* L, const double* sc, hipStream_t s)
+// One iteration of the CG on grid 0's dense vectors: x in d_Z, r in mg[0].r, ap in d_AP, the direction in d_Pv
+// and d_R in turn (it even: from d_Pv into d_R), z = V(r).
+static int mg_cg_iteration(cmp_level* L, int it, int maxit, double inv_n, hipStream_t s)
+{
+    const int dim = L->P.dim, nb = cmp::mg_blocks(L->mg[0].G.nc);
+    double* p = (it & 1) ? L->d_Pv : L->d_R;
+    double* pap = L->d_part + nb;   // (beside the first slot, which takes r.r)
+    cmp::MgArgs a = mg_args(L, L->d_sc);
+    a.scw = L->d_sc;
+    a.G = L->mg[0].G;
+    for (int d = 0; d < 3; ++d) a.b[d] = L->mg[0].b[d];
+    a.inv_n = inv_n;
+    a.maxit = (double)maxit;
+    a.src = L->mg[0].x[L->mg[0].cur];
+    a.r = (it & 1) ? L->d_R : L->d_Pv;
+    a.dst = p;
+    a.rw = L->d_AP;
+    a.part = pap;
+    int r = mg_launch(dim, cmp::MG_CG_AP, a, s);
+    if (r) return r;
+    if (nb > 1024) CMP_TRY(launch_reduce_sums(pap, nb, 1, L->d_sc + CG_PAP, s, L->d_sc));
+    a.src = p;
+    a.id = L->d_AP;
+    a.dst = L->d_Z;
+    a.rw = L->mg[0].r;
+    a.r = pap;
+    a.part = L->d_part;
+    r = mg_launch(dim, cmp::MG_CG_XR, a, s);
+    if (!r) r = mg_vcycle(L, L->d_sc, 0, s, L->d_part);
+    if (!r) r = mg_launch(dim, cmp::MG_CG_END, a, s);
+    return r;
+}
+
+// the CG's vectors from cg_init's box layout (r, x = 0), z = V(r), the first sums
+static int mg_cg_start(cmp_level* L, double inv_n, hipStream_t s)
 {
     const int dim = L->P.dim;
-    cmp::MgArgs a = mg_args(L, sc);
+    CMP_TRY(launch_reduce_sums(L->d_part, L->nblocks, 1, L->d_sc + CG_RR, s));
+    cmp::MgArgs a = mg_args(L, nullptr);
     a.G = L->mg[0].G;
     a.src = L->d_R;
     a.dst = L->mg[0].r;
     int r = mg_launch(dim, cmp::MG_GATHER_R, a, s);
-    if (!r) r = mg_vcycle(L, sc, 0, s);
-    if (r) return r;
-    a.src = L->mg[0].x[L->mg[0].cur];
+    a.src = L->d_X;
     a.dst = L->d_Z;
-    a.r = L->d_R;
+    if (!r) r = mg_launch(dim, cmp::MG_GATHER_R, a, s);
+    if (!r) r = mg_vcycle(L, nullptr, 0, s, L->d_part);
+    a.scw = L->d_sc;
     a.part = L->d_part;
-    return mg_launch(dim, cmp::MG_CG_RZ, a, s);
+    a.inv_n = inv_n;
+    a.first = 1;
+    return r ? r : mg_launch(dim, cmp::MG_CG_END, a, s);
 }
 
 extern "C" {
@@ -1535,37 +1584,33 @@ static int pf_gradq_implicit(cmp_level* L, double dt, double eta, double* gradq,
     const bool mg = !L->mg.empty();
     const double inv_n = mg ? 1.0 / (double)L->ncell : 0.0;
     if (mg) {
-        // the V-cycle's face coefficients and diagonals for this b, then z = V(r)
+        // the V-cycle's face coefficients and diagonals for this b
         int r = mg_prepare(L, s);
-        if (!r) r = mg_precondition(L, nullptr, s);
+        if (!r) r = mg_cg_start(L, inv_n, s);
         if (r) return r;
-    }
-    CMP_TRY(launch_reduce_sums(L->d_part, L->nblocks, mg ? 4 : 2, sc + CG_RR, s, nullptr, sc + CG_ZS));
-    if (mg) {
-        // p = z - mean(z)
-        CMP_TRY(launch_cg_start(sc, s, inv_n));
-        CMP_TRY(launch_cg_p(dim, L->pg, L->maxcells, sc, L->d_Z, L->d_Pv, s, inv_n, nullptr, 1));
     } else {
+        CMP_TRY(launch_reduce_sums(L->d_part, L->nblocks, 2, sc + CG_RR, s));
         CMP_TRY(launch_cg_start(sc, s));
     }
     // the host looks at the stop flag every `chunk` iterations; iterations queued past the stop
     // return at once. A chunk's launches depend only on the level's buffers, so it is captured once
-    // into a graph and replayed (one launch instead of 60-80 per iteration).
+    // into a graph and replayed (an even number of iterations: the direction's two buffers take turns).
     const int chunk = mg ? 8 : 16;
     auto enqueue_chunk = [&](hipStream_t cs) -> int {
         for (int q = 0; q < chunk; ++q) {
+            if (mg) {
+                const int r = mg_cg_iteration(L, q, maxit, inv_n, cs);
+                if (r) return r;
+                continue;
+            }
             CMP_TRY(launch_fill(dim, 1, L->fdA, L->nghost1, L->d_Pv, L->d_err, cs));
             CMP_TRY(launch_cg_ap(dim, L->pg, L->maxcells, sc, L->d_Bf, L->d_Pv, L->d_AP, L->d_part, cs));
             CMP_TRY(launch_reduce_sums(L->d_part, L->nblocks, 1, sc + CG_PAP, cs, sc));
-            CMP_TRY(launch_cg_xr(dim, L->pg, L->maxcells, sc, mg ? nullptr : L->d_ID, L->d_X, L->d_R, L->d_Z,
-                                 L->d_Pv, L->d_AP, L->d_part, cs));
-            if (mg) {
-                int r = mg_precondition(L, sc, cs);
-                if (r) return r;
-            }
-            CMP_TRY(launch_reduce_sums(L->d_part, L->nblocks, mg ? 4 : 2, sc + CG_RRNEW, cs, sc, sc + CG_ZS));
-            CMP_TRY(launch_cg_p(dim, L->pg, L->maxcells, sc, L->d_Z, L->d_Pv, cs, inv_n));
-            CMP_TRY(launch_cg_end(sc, maxit, cs, inv_n));
+            CMP_TRY(launch_cg_xr(dim, L->pg, L->maxcells, sc, L->d_ID, L->d_X, L->d_R, L->d_Z, L->d_Pv, L->d_AP,
+                                 L->d_part, cs));
+            CMP_TRY(launch_reduce_sums(L->d_part, L->nblocks, 2, sc + CG_RRNEW, cs, sc));
+            CMP_TRY(launch_cg_p(dim, L->pg, L->maxcells, sc, L->d_Z, L->d_Pv, cs));
+            CMP_TRY(launch_cg_end(sc, maxit, cs));
         }
         return CMP_OK;
     };
@@ -1596,6 +1641,14 @@ static int pf_gradq_implicit(cmp_level* L, double dt, double eta, double* gradq,
         if (queued > maxit) return CMP_ERR_NAN;   // the device stop test failed to fire
     }
     L->cg_iters = (int)L->h_pin[3];
+    if (mg) {
+        cmp::MgArgs a = mg_args(L, nullptr);
+        a.G = L->mg[0].G;
+        a.src = L->d_Z;
+        a.dst = L->d_X;
+        const int r = mg_launch(dim, cmp::MG_SCATTER, a, s);
+        if (r) return r;
+    }
     CMP_TRY(launch_fill(dim, 1, L->fdA, L->nghost1, L->d_X, L->d_err, s));
     CMP_TRY(launch_pf_gradx(dim, L->pg, L->maxfaces, L->d_X, gradq, L->d_bits + 1, L->d_boxflag, s));
     return CMP_OK;

@@ -318,7 +318,8 @@ struct MgGrid {
 };
 
 enum MgOp {
-    MG_GATHER_R, MG_GATHER_B, MG_RESTRICT_B, MG_DIAG, MG_SMOOTH, MG_RESID_RESTRICT, MG_BOTTOM, MG_CG_RZ
+    MG_GATHER_R, MG_SCATTER, MG_GATHER_B, MG_RESTRICT_B, MG_DIAG, MG_SMOOTH, MG_RESID_RESTRICT, MG_BOTTOM, MG_CG_RZ,
+    MG_CG_SUMS, MG_CG_AP, MG_CG_XR, MG_CG_END
 };
 
 // Arguments of one multigrid operation (the fields an operation does not use are ignored):
@@ -326,8 +327,12 @@ enum MgOp {
 //   RESTRICT_B: b[d] (G) -> bc[d] (Gc); DIAG: b -> dst = 1/diag; SMOOTH: dst = x + omega id (r - A x),
 //   x as `from` says (src, zero swept once, src plus xc on Gc); RESID_RESTRICT: dst (Gc) = mean of the
 //   children of r - A src (G); BOTTOM: dst = `sweeps` Jacobi sweeps from 0 on r (G at most 1024 cells);
-//   CG_RZ: partials of r.z, z and r into part's second to fourth slots, r and dst (= z) in box layout; z
-//   taken from src (dense G) into dst first when src is non-null.
+//   SCATTER: src (dense G) -> dst (box layout); CG_RZ: partials of r.z, z and r into part's second to
+//   fourth slots, r and dst (= z) in box layout.
+// The iteration of a CG whose vectors are dense on G, mg_blocks(G.nc) partials a slot: SMOOTH with part and
+//   CG_SUMS (src = z): partials of r.z, z and r as CG_RZ's; CG_AP: p (dst) = z' + beta p_old, z' = src -
+//   mean, p_old = r, ap (rw) of it, partials of p.ap; CG_XR: x (dst) += al p (src), r (rw) -= al ap (id),
+//   partials of r.r, p.ap from its partials r (another slot than part); CG_END: the four sums, then the iteration's end (first: the solve's start, r.r known).
 enum MgFrom { MG_FROM_X = 0, MG_FROM_ZERO = 1, MG_FROM_COARSE = 2 };
 struct MgArgs {
     PfGeom g;
@@ -343,10 +348,21 @@ struct MgArgs {
     double* part;
     MgGrid G, Gc;
     const double* xc;
+    double* rw;
+    double* scw;
+    double inv_n, maxit;
+    int first;
     double omega;
     int from;
     int sweeps;
 };
+
+// blocks of a dense grid's kernels (and so partials of a sum)
+inline int mg_blocks(long long n)
+{
+    const long long b = (n + NT - 1) / NT;
+    return (int)(b > 65536 ? 65536 : b < 1 ? 1 : b);
+}
 
 template <int DIM>
 hipError_t launch_mg_dim(int op, const MgArgs& a, hipStream_t s);
@@ -522,6 +538,7 @@ enum {
     CG_SUM = 10,    // two slots for level sums (CAC's sum mech, sum W; the mean of the rhs)
     CG_ZS = 12,     // sum of z over the unknowns (the preconditioned residual's constant part)
     CG_RS = 13,     // sum of r over the unknowns; the pair is reduced together
+    CG_BETA = 14,   // r.z over the iteration before's: the next direction's coefficient (0: the first)
     CG_NSC = 16
 };
 // r.z of the residual against the projected z - mean(z) when inv_n = 1/(number of unknowns) > 0:
@@ -529,6 +546,45 @@ enum {
 __host__ __device__ inline double cg_rz_projected(const double* sc, int slot, double inv_n)
 {
     return (inv_n > 0.0) ? sc[slot] - sc[CG_ZS] * inv_n * sc[CG_RS] : sc[slot];
+}
+// the initial r.r and r.z (projected with inv_n > 0) start the stopping test (one thread)
+__device__ inline void cg_start_step(double* sc, double inv_n)
+{
+    sc[CG_RZ] = cg_rz_projected(sc, CG_RZ, inv_n);
+    const double rr = sc[CG_RR];
+    sc[CG_B2] = rr;
+    sc[CG_BEST] = rr;
+    sc[CG_STALL] = 0.0;
+    sc[CG_IT] = 0.0;
+    sc[CG_BETA] = 0.0;
+    sc[CG_DONE] = (rr > 0.0 && sc[CG_RZ] > 0.0) ? 0.0 : 1.0;   // a zero (or NaN) right-hand side: x = 0
+}
+// the end of an iteration (one thread): pAp <= 0 stops without counting it; r.r <= 1e-28 b.b, 400
+// iterations without a new minimum of r.r (CG's residual norm is not monotone and can plateau for tens of
+// iterations before it falls again) or maxit stop after it
+__device__ inline void cg_end_step(double* sc, double maxit, double inv_n)
+{
+    if (!(sc[CG_PAP] > 0.0)) {
+        sc[CG_DONE] = 1.0;
+        return;
+    }
+    const double rr = sc[CG_RRNEW], rz = cg_rz_projected(sc, CG_RZNEW, inv_n);
+    sc[CG_RR] = rr;
+    sc[CG_BETA] = rz / sc[CG_RZ];
+    sc[CG_RZ] = rz;
+    const double it = sc[CG_IT] + 1.0;
+    sc[CG_IT] = it;
+    bool done = false;
+    if (rr < sc[CG_BEST]) {
+        sc[CG_BEST] = rr;
+        sc[CG_STALL] = 0.0;
+    } else {
+        const double st = sc[CG_STALL] + 1.0;
+        sc[CG_STALL] = st;
+        done = st > 400.0;
+    }
+    if (!(rr > 1.0e-28 * sc[CG_B2]) || !(it < maxit)) done = true;
+    if (done) sc[CG_DONE] = 1.0;
 }
 // ap = -div(b grad p) (p ghosts filled; Neumann domain faces carry no flux), partial of p.ap
 hipError_t launch_cg_ap(int dim, const PfGeom& g, long long maxcells, const double* sc, const double* Bf,
@@ -547,10 +603,10 @@ hipError_t launch_cg_end(double* sc, int maxit, hipStream_t s, double inv_n = 0.
 // face gradient of x (ghosts filled), zero on Neumann domain faces, with max |.|
 hipError_t launch_pf_gradx(int dim, const PfGeom& g, const long long* maxfaces, const double* X,
                            double* gq, unsigned long long* gmax_bits, int* boxflag, hipStream_t s);
-// sums[v] = the sum of the nblocks partials of value v (fixed order), values 2 and 3 into sums2[0] and
-// sums2[1]; sc non-null: nothing once the CG's stop flag sc[CG_DONE] is set
+// sums[v] = the sum of the nblocks partials of value v (fixed order); sc non-null: nothing once the
+// CG's stop flag sc[CG_DONE] is set
 hipError_t launch_reduce_sums(const double* part, int nblocks, int nvals, double* sums, hipStream_t s,
-                              const double* sc = nullptr, double* sums2 = nullptr);
+                              const double* sc = nullptr);
 // The partial sums of every level of a composite solve in one launch: per level the same fixed-order
 // reduction as launch_reduce_sums (into per[l * nvals + v]), then sums[v] = the levels' values added
 // in level order.

@@ -57,7 +57,7 @@ namespace cmp {
 // of every grid from the level's d_Bf, and one V-cycle from grid m's residual (its result in
 // mg[m].x[mg[m].cur])
 int mg_prepare(cmp_level* L, hipStream_t s);
-int mg_vcycle(cmp_level* L, const double* sc, size_t m, hipStream_t s);
+int mg_vcycle(cmp_level* L, const double* sc, size_t m, hipStream_t s, double* part = nullptr);
 }  // namespace cmp
 
 struct cmp_level {

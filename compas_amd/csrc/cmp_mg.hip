@@ -29,6 +29,26 @@ __device__ __forceinline__ double mg_wave_sum(double v)
     return v;
 }
 
+// the block's sums of N values a thread -> part[m * nb + block]
+template <int N>
+__device__ __forceinline__ void mg_block_sums(const double (&w)[N], double* part, long long nb, long long blk)
+{
+    __shared__ double red[N][NT / 64];
+#pragma unroll
+    for (int m = 0; m < N; ++m) {
+        const double t = mg_wave_sum(w[m]);
+        if ((threadIdx.x & 63) == 0) red[m][threadIdx.x >> 6] = t;
+    }
+    __syncthreads();
+    if (threadIdx.x < N) {
+        const int m = threadIdx.x;
+        double s = red[m][0];
+#pragma unroll
+        for (int v = 1; v < NT / 64; ++v) s += red[m][v];
+        part[m * nb + blk] = s;
+    }
+}
+
 template <int DIM>
 __device__ __forceinline__ void mg_cell(const MgGrid& G, long long q, int& i, int& j, int& k)
 {
@@ -97,6 +117,22 @@ __global__ __launch_bounds__(NT) void k_mg_gather_r(PfGeom g, const double* __re
     j += ab.lo[1];
     k += ab.lo[2];
     r0[mg_idx(G, i - g.dlo[0], j - g.dlo[1], (DIM == 3) ? k - g.dlo[2] : 0)] = R[ab.off + fab_index(ab, i, j, k)];
+}
+
+template <int DIM>
+__global__ __launch_bounds__(NT) void k_mg_scatter(PfGeom g, const double* __restrict__ x0, double* X, MgGrid G)
+{
+    long long q;
+    const BoxDev ab = g.abox[cell_block(g.cmap, q)];
+    const int n0 = ab.hi[0] - ab.lo[0] + 1, n1 = ab.hi[1] - ab.lo[1] + 1;
+    const int n2 = (DIM == 3) ? ab.hi[2] - ab.lo[2] + 1 : 1;
+    if (q >= (long long)n0 * n1 * n2) return;
+    int i, j, k;
+    pos3(q, n0, n1, i, j, k);
+    i += ab.lo[0];
+    j += ab.lo[1];
+    k += ab.lo[2];
+    X[ab.off + fab_index(ab, i, j, k)] = x0[mg_idx(G, i - g.dlo[0], j - g.dlo[1], (DIM == 3) ? k - g.dlo[2] : 0)];
 }
 
 // the box face buffer of direction D (cmp_face_layout, one component) -> the dense face array
@@ -168,15 +204,15 @@ __global__ __launch_bounds__(NT) void k_mg_diag(const double* __restrict__ b0, c
 // one damped Jacobi sweep y = x + omega D^-1 (r - A x). FROM: x the array (MG_FROM_X), the sweep from zero
 // omega D^-1 r (MG_FROM_ZERO) or the array plus the coarser grid's value at the parent cell
 // (MG_FROM_COARSE), the last two computed where they are read: a launch and a pass over memory each against
-// one or two more loads a neighbour, all from cache: four launches a
-// grid instead of six. With one launch for z's scatter and the sums and one for four sums, a 512 x 256 Grad_Q
-// 2.68 -> 2.31 ms, eight cases' CAC steps 7.90 -> 6.92 ms.
-template <int DIM, int FROM>
+// one or two more loads a neighbour, all from cache: four launches a grid instead of six. SUMS: the last
+// sweep of a CG's preconditioner adds up r.z, z and r as it goes.
+template <int DIM, int FROM, bool SUMS>
 __global__ __launch_bounds__(NT) void k_mg_smooth(const double* __restrict__ sc, const double* __restrict__ x,
                                                   double* __restrict__ y, const double* __restrict__ r,
                                                   const double* __restrict__ b0, const double* __restrict__ b1,
                                                   const double* __restrict__ b2, const double* __restrict__ id,
-                                                  MgGrid G, double omega, const double* __restrict__ xc, MgGrid Gc)
+                                                  MgGrid G, double omega, const double* __restrict__ xc, MgGrid Gc,
+                                                  double* part)
 {
     if (sc && sc[CG_DONE] != 0.0) return;
     const double* b[3] = {b0, b1, b2};
@@ -188,11 +224,19 @@ __global__ __launch_bounds__(NT) void k_mg_smooth(const double* __restrict__ sc,
         if (FROM == MG_FROM_COARSE) return x[c] + xc[mg_idx(Gc, i >> 1, j >> 1, (DIM == 3) ? (k >> 1) : 0)];
         return x[c];
     };
+    double w[3] = {0.0, 0.0, 0.0};
     for (long long q = (long long)blockIdx.x * NT + threadIdx.x; q < G.nc; q += (long long)gridDim.x * NT) {
         int i, j, k;
         mg_cell<DIM>(G, q, i, j, k);
-        y[q] = value(i, j, k) + omega * id[q] * (r[q] - mg_apply<DIM>(G, value, b, i, j, k));
+        const double z = value(i, j, k) + omega * id[q] * (r[q] - mg_apply<DIM>(G, value, b, i, j, k));
+        y[q] = z;
+        if (SUMS) {
+            w[0] += r[q] * z;
+            w[1] += z;
+            w[2] += r[q];
+        }
     }
+    if (SUMS) mg_block_sums(w, part + gridDim.x, gridDim.x, blockIdx.x);
 }
 
 // rc = mean over the 2^DIM children of (r - A x)
@@ -518,10 +562,10 @@ __global__ __launch_bounds__(NTAIL) void k_mg_tail(MgTail t)
 }
 
 // the partial sums of one CG iteration's r.z, sum z and sum r (the second, third and fourth partial
-// slots; the first holds r.r). x0 non-null: z is the dense grid's value there, written to Z on the way.
+// slots; the first holds r.r)
 template <int DIM>
 __global__ __launch_bounds__(NT) void k_cg_rz(PfGeom g, const double* __restrict__ sc, const double* __restrict__ R,
-                                              const double* __restrict__ x0, double* Z, MgGrid G, double* part)
+                                              const double* __restrict__ Z, double* part)
 {
     if (sc && sc[CG_DONE] != 0.0) return;
     long long q;
@@ -536,42 +580,155 @@ __global__ __launch_bounds__(NT) void k_cg_rz(PfGeom g, const double* __restrict
         j += ab.lo[1];
         k += ab.lo[2];
         const long long c = ab.off + fab_index(ab, i, j, k);
-        double z;
-        if (x0) {
-            z = x0[mg_idx(G, i - g.dlo[0], j - g.dlo[1], (DIM == 3) ? k - g.dlo[2] : 0)];
-            Z[c] = z;
-        } else {
-            z = Z[c];
-        }
-        const double r = R[c];
+        const double r = R[c], z = Z[c];
         w[0] = r * z;
         w[1] = z;
         w[2] = r;
     }
-    __shared__ double red[3][NT / 64];
-#pragma unroll
-    for (int m = 0; m < 3; ++m) {
-        const double t = mg_wave_sum(w[m]);
-        if ((threadIdx.x & 63) == 0) red[m][threadIdx.x >> 6] = t;
-    }
-    __syncthreads();
-    if (threadIdx.x < 3) {
-        const int m = threadIdx.x;
-        double s = red[m][0];
-#pragma unroll
-        for (int v = 1; v < NT / 64; ++v) s += red[m][v];
-        const long long nb = (long long)gridDim.x * gridDim.y;
-        part[(m + 1) * nb + (long long)blockIdx.y * gridDim.x + blockIdx.x] = s;
-    }
+    const long long nb = (long long)gridDim.x * gridDim.y;
+    mg_block_sums(w, part + nb, nb, (long long)blockIdx.y * gridDim.x + blockIdx.x);
 }
 
-dim3 mg_grid(long long n)
+// ---- the iteration of a CG on one dense grid (a level that covers its domain) -------------------------
+// Bound by its launches on all but the largest levels: on the dense arrays there are no ghost cells to fill,
+// nothing to gather for or scatter from the V-cycle, and the direction's update is taken where ap reads it
+// (p_old -> p, two arrays in turn), so that an iteration outside the V-cycle has three launches (four above
+// 1024 partials a sum) where the box layout's had nine (eight cases' CAC steps 6.90 -> 5.55 ms).
+
+// the partials of r.z, z and r (a preconditioner whose last launch is not a sweep of grid 0)
+__global__ __launch_bounds__(NT) void k_dcg_sums(const double* __restrict__ sc, const double* __restrict__ r,
+                                                 const double* __restrict__ z, long long nc, double* part)
 {
-    long long b = (n + NT - 1) / NT;
-    if (b > 65536) b = 65536;
-    if (b < 1) b = 1;
-    return dim3((unsigned)b);
+    if (sc && sc[CG_DONE] != 0.0) return;
+    double w[3] = {0.0, 0.0, 0.0};
+    for (long long q = (long long)blockIdx.x * NT + threadIdx.x; q < nc; q += (long long)gridDim.x * NT) {
+        w[0] += r[q] * z[q];
+        w[1] += z[q];
+        w[2] += r[q];
+    }
+    mg_block_sums(w, part + gridDim.x, gridDim.x, blockIdx.x);
 }
+
+// p = z - mean(z) + beta p_old; ap = -div(b grad p) with the box layout's arithmetic (k_cg_ap); partials of p.ap
+template <int DIM>
+__global__ __launch_bounds__(NT) void k_dcg_ap(const double* __restrict__ sc, const double* __restrict__ z,
+                                               const double* __restrict__ pold, double* __restrict__ p,
+                                               double* __restrict__ AP, const double* __restrict__ b0,
+                                               const double* __restrict__ b1, const double* __restrict__ b2,
+                                               MgGrid G, double dx0, double dx1, double dx2, double inv_n, double* part)
+{
+    if (sc[CG_DONE] != 0.0) return;
+    const double be = sc[CG_BETA], zm = sc[CG_ZS] * inv_n;
+    const double* b[3] = {b0, b1, b2};
+    const double dx[3] = {dx0, dx1, dx2};
+    auto value = [&](int i, int j, int k) __attribute__((always_inline)) -> double {
+        const long long c = mg_idx(G, i, j, k);
+        const double zc = z[c] - zm;
+        return be != 0.0 ? fma(be, pold[c], zc) : zc;   // (the first direction: p_old holds nothing)
+    };
+    double w[1] = {0.0};
+    for (long long q = (long long)blockIdx.x * NT + threadIdx.x; q < G.nc; q += (long long)gridDim.x * NT) {
+        int i, j, k;
+        mg_cell<DIM>(G, q, i, j, k);
+        const int co[3] = {i, j, k};
+        const double pc = value(i, j, k);
+        double acc = 0.0;
+#pragma unroll
+        for (int d = 0; d < DIM; ++d) {
+            int m[3] = {i, j, k}, n[3] = {i, j, k}, f[3] = {i, j, k};
+            const bool lo = co[d] == 0, hi = co[d] == G.n[d] - 1;
+            m[d] = lo ? G.n[d] - 1 : co[d] - 1;
+            n[d] = hi ? 0 : co[d] + 1;
+            f[d] += 1;
+            const double fp = (hi && !G.periodic[d])
+                                  ? 0.0
+                                  : b[d][mg_face(G, d, f[0], f[1], f[2])] * (value(n[0], n[1], n[2]) - pc) / dx[d];
+            const double fm = (lo && !G.periodic[d])
+                                  ? 0.0
+                                  : b[d][mg_face(G, d, i, j, k)] * (pc - value(m[0], m[1], m[2])) / dx[d];
+            const double t = (fp - fm) / dx[d];
+            acc = (d == 0) ? t : acc + t;
+        }
+        p[q] = pc;
+        AP[q] = -acc;
+        w[0] += pc * (-acc);
+    }
+    mg_block_sums(w, part, gridDim.x, blockIdx.x);
+}
+
+// x += al p, r -= al ap, partials of r.r into the first slot. nred > 0: p.ap is its nred partials' sum, taken
+// by every block in the same order (a launch less; at most 1024 values, four a thread); else it is in sc.
+__global__ __launch_bounds__(NT) void k_dcg_xr(double* __restrict__ sc, double* __restrict__ x,
+                                               double* __restrict__ r, const double* __restrict__ p,
+                                               const double* __restrict__ AP, long long nc, int nred,
+                                               const double* __restrict__ pap_part, double* part)
+{
+    if (sc[CG_DONE] != 0.0) return;
+    __shared__ double red[NT / 64];
+    double pap;
+    if (nred > 0) {
+        double t = 0.0;
+        for (int b = threadIdx.x; b < nred; b += NT) t += pap_part[b];
+        t = mg_wave_sum(t);
+        if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = t;
+        __syncthreads();
+        pap = red[0];
+#pragma unroll
+        for (int v = 1; v < NT / 64; ++v) pap += red[v];
+        if (blockIdx.x == 0 && threadIdx.x == 0) sc[CG_PAP] = pap;
+    } else {
+        pap = sc[CG_PAP];
+    }
+    if (!(pap > 0.0)) return;
+    const double al = sc[CG_RZ] / pap;
+    double w[1] = {0.0};
+    for (long long q = (long long)blockIdx.x * NT + threadIdx.x; q < nc; q += (long long)gridDim.x * NT) {
+        x[q] += al * p[q];
+        const double v = r[q] - al * AP[q];
+        r[q] = v;
+        w[0] += v * v;
+    }
+    mg_block_sums(w, part, gridDim.x, blockIdx.x);
+}
+
+// the four sums of an iteration in one workgroup, then its end; first: r.z and the means' sums alone (r.r of the
+// initial residual is in sc), then the solve's start
+__global__ __launch_bounds__(1024) void k_dcg_end(double* sc, const double* __restrict__ part, int nb, double maxit,
+                                                  double inv_n, int first)
+{
+    if (!first && sc[CG_DONE] != 0.0) return;
+    __shared__ double red[4][16];
+    const int tid = threadIdx.x;
+    double w[4] = {0.0, 0.0, 0.0, 0.0};
+    for (int b = tid; b < nb; b += 1024) {
+#pragma unroll
+        for (int m = 0; m < 4; ++m)
+            if (m > 0 || !first) w[m] += part[(long long)m * nb + b];
+    }
+#pragma unroll
+    for (int m = 0; m < 4; ++m) {
+        const double t = mg_wave_sum(w[m]);
+        if ((tid & 63) == 0) red[m][tid >> 6] = t;
+    }
+    __syncthreads();
+    if (tid != 0) return;
+#pragma unroll
+    for (int m = 0; m < 4; ++m) {
+        w[m] = red[m][0];
+#pragma unroll
+        for (int v = 1; v < 16; ++v) w[m] += red[m][v];
+    }
+    if (!first) sc[CG_RRNEW] = w[0];
+    sc[first ? CG_RZ : CG_RZNEW] = w[1];
+    sc[CG_ZS] = w[2];
+    sc[CG_RS] = w[3];
+    if (first)
+        cg_start_step(sc, inv_n);
+    else
+        cg_end_step(sc, maxit, inv_n);
+}
+
+dim3 mg_grid(long long n) { return dim3((unsigned)mg_blocks(n)); }
 
 dim3 box_grid(long long maxn, int nbox)
 {
@@ -610,10 +767,13 @@ hipError_t launch_mg_dim(int op, const MgArgs& a, hipStream_t s)
         hipLaunchKernelGGL((k_mg_diag<DIM>), mg_grid(a.G.nc), dim3(NT), 0, s, a.b[0], a.b[1], a.b[2], a.dst, a.G);
         break;
     case MG_SMOOTH: {
-        const auto f = a.from == MG_FROM_X ? k_mg_smooth<DIM, MG_FROM_X>
-                       : a.from == MG_FROM_ZERO ? k_mg_smooth<DIM, MG_FROM_ZERO> : k_mg_smooth<DIM, MG_FROM_COARSE>;
+        if (a.part && a.from != MG_FROM_X) return hipErrorInvalidValue;
+        const auto f = a.part                    ? k_mg_smooth<DIM, MG_FROM_X, true>
+                       : a.from == MG_FROM_X    ? k_mg_smooth<DIM, MG_FROM_X, false>
+                       : a.from == MG_FROM_ZERO ? k_mg_smooth<DIM, MG_FROM_ZERO, false>
+                                                : k_mg_smooth<DIM, MG_FROM_COARSE, false>;
         hipLaunchKernelGGL(f, mg_grid(a.G.nc), dim3(NT), 0, s, a.sc, a.src, a.dst, a.r, a.b[0], a.b[1], a.b[2],
-                           a.id, a.G, a.omega, a.xc, a.Gc);
+                           a.id, a.G, a.omega, a.xc, a.Gc, a.part);
         break;
     }
     case MG_RESID_RESTRICT:
@@ -625,9 +785,30 @@ hipError_t launch_mg_dim(int op, const MgArgs& a, hipStream_t s)
         hipLaunchKernelGGL((k_mg_bottom<DIM>), dim3(1), dim3(1024), 0, s, a.sc, a.r, a.dst, a.b[0], a.b[1], a.b[2],
                            a.id, a.G, a.omega, a.sweeps);
         break;
+    case MG_SCATTER:
+        hipLaunchKernelGGL((k_mg_scatter<DIM>), cell_grid(a.g.cmap, a.g.ncmap, a.maxcells, a.g.nbox), dim3(NT), 0, s,
+                           a.g, a.src, a.dst, a.G);
+        break;
     case MG_CG_RZ:
         hipLaunchKernelGGL((k_cg_rz<DIM>), cell_grid(a.g.cmap, a.g.ncmap, a.maxcells, a.g.nbox), dim3(NT), 0, s, a.g,
-                           a.sc, a.r, a.src, a.dst, a.G, a.part);
+                           a.sc, a.r, a.dst, a.part);
+        break;
+    case MG_CG_SUMS:
+        hipLaunchKernelGGL(k_dcg_sums, mg_grid(a.G.nc), dim3(NT), 0, s, a.sc, a.r, a.src, a.G.nc, a.part);
+        break;
+    case MG_CG_AP:
+        hipLaunchKernelGGL((k_dcg_ap<DIM>), mg_grid(a.G.nc), dim3(NT), 0, s, a.sc, a.src, a.r, a.dst, a.rw, a.b[0],
+                           a.b[1], a.b[2], a.G, a.g.dx[0], a.g.dx[1], a.g.dx[2], a.inv_n, a.part);
+        break;
+    case MG_CG_XR: {
+        const int nb = mg_blocks(a.G.nc);
+        hipLaunchKernelGGL(k_dcg_xr, mg_grid(a.G.nc), dim3(NT), 0, s, a.scw, a.dst, a.rw, a.src, a.id, a.G.nc,
+                           nb <= 1024 ? nb : 0, a.r, a.part);
+        break;
+    }
+    case MG_CG_END:
+        hipLaunchKernelGGL(k_dcg_end, dim3(1), dim3(1024), 0, s, a.scw, a.part, mg_blocks(a.G.nc), a.maxit, a.inv_n,
+                           a.first);
         break;
     default:
         return hipErrorInvalidValue;

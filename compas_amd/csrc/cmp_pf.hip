@@ -804,15 +804,14 @@ __device__ __forceinline__ double reduce_block_parts(const double* __restrict__ 
     return u;
 }
 
-// (the sums from the third on go to sums2)
 __global__ __launch_bounds__(NRED) void k_reduce_sums(const double* __restrict__ part, int nblocks, double* sums,
-                                                      double* sums2, const double* __restrict__ sc)
+                                                      const double* __restrict__ sc)
 {
     if (sc && sc[CG_DONE] != 0.0) return;
     __shared__ double red[NRED / 64];
     const int v = blockIdx.x;
     const double u = reduce_block_parts(part + (long long)v * nblocks, nblocks, red);
-    if (threadIdx.x == 0) *(v < 2 ? sums + v : sums2 + (v - 2)) = u;
+    if (threadIdx.x == 0) sums[v] = u;
 }
 
 // every level's sums (per[l * nvals + v], as k_reduce_sums leaves them) and their sum in level order
@@ -836,45 +835,18 @@ __global__ __launch_bounds__(NRED) void k_reduce_levels(LevelParts lp, int nvals
 
 // CG bookkeeping on the device, so that the iteration stops where the host loop of the solve's
 // restatement stops without a host round trip per iteration: start after r.r of the initial
-// residual landed in sc[CG_RR]; end after each iteration (pAp <= 0 stops without counting it;
-// r.r <= 1e-28 b.b, 400 iterations without a new minimum of r.r (CG's residual norm is not monotone
-// and can plateau for tens of iterations before it falls again) or maxit stop after it).
+// residual landed in sc[CG_RR]; end after each iteration.
 __global__ void k_cg_start(double* sc, double inv_n)
 {
     if (threadIdx.x != 0 || blockIdx.x != 0) return;
-    sc[CG_RZ] = cg_rz_projected(sc, CG_RZ, inv_n);
-    const double rr = sc[CG_RR];
-    sc[CG_B2] = rr;
-    sc[CG_BEST] = rr;
-    sc[CG_STALL] = 0.0;
-    sc[CG_IT] = 0.0;
-    sc[CG_DONE] = (rr > 0.0 && sc[CG_RZ] > 0.0) ? 0.0 : 1.0;   // a zero (or NaN) right-hand side: x = 0
+    cg_start_step(sc, inv_n);
 }
 
 __global__ void k_cg_end(double* sc, double maxit, double inv_n)
 {
     if (threadIdx.x != 0 || blockIdx.x != 0) return;
     if (sc[CG_DONE] != 0.0) return;
-    if (!(sc[CG_PAP] > 0.0)) {
-        sc[CG_DONE] = 1.0;
-        return;
-    }
-    const double rr = sc[CG_RRNEW];
-    sc[CG_RR] = rr;
-    sc[CG_RZ] = cg_rz_projected(sc, CG_RZNEW, inv_n);
-    const double it = sc[CG_IT] + 1.0;
-    sc[CG_IT] = it;
-    bool done = false;
-    if (rr < sc[CG_BEST]) {
-        sc[CG_BEST] = rr;
-        sc[CG_STALL] = 0.0;
-    } else {
-        const double st = sc[CG_STALL] + 1.0;
-        sc[CG_STALL] = st;
-        done = st > 400.0;
-    }
-    if (!(rr > 1.0e-28 * sc[CG_B2]) || !(it < maxit)) done = true;
-    if (done) sc[CG_DONE] = 1.0;
+    cg_end_step(sc, maxit, inv_n);
 }
 
 hipError_t launch_reduce_levels(const LevelParts& lp, int nvals, double* per, double* sums, hipStream_t s,
@@ -886,10 +858,9 @@ hipError_t launch_reduce_levels(const LevelParts& lp, int nvals, double* per, do
 }
 
 hipError_t launch_reduce_sums(const double* part, int nblocks, int nvals, double* sums, hipStream_t s,
-                              const double* sc, double* sums2)
+                              const double* sc)
 {
-    if (nvals > 2 && !sums2) return hipErrorInvalidValue;
-    hipLaunchKernelGGL(k_reduce_sums, dim3(nvals), dim3(NRED), 0, s, part, nblocks, sums, sums2, sc);
+    hipLaunchKernelGGL(k_reduce_sums, dim3(nvals), dim3(NRED), 0, s, part, nblocks, sums, sc);
     return hipGetLastError();
 }
 
