@@ -1481,6 +1481,21 @@ int cmp::mg_vcycle(cmp_level* L, const double* sc, size_t m, hipStream_t s, doub
         if ((r = mg_launch(dim, cmp::MG_BOTTOM, a, s))) return r;
         return part ? mg_sums(L, sc, m, part, s) : CMP_OK;
     }
+    if (dim == 2) {
+        // two launches a grid (every extent is even: a coarser grid exists)
+        auto& C = L->mg[m + 1];
+        a.Gc = C.G;
+        a.dst = V.x[1];
+        a.rw = C.r;
+        if ((r = mg_launch(dim, cmp::MG_DOWN, a, s))) return r;
+        if ((r = mg_vcycle(L, sc, m + 1, s))) return r;
+        a.src = V.x[1];
+        a.xc = C.x[C.cur];
+        a.dst = V.x[0];
+        if ((r = mg_launch(dim, cmp::MG_UP, a, s))) return r;
+        V.cur = 0;
+        return part ? mg_sums(L, sc, m, part, s) : CMP_OK;
+    }
     a.from = cmp::MG_FROM_ZERO;
     a.dst = V.x[1];
     if ((r = mg_launch(dim, cmp::MG_SMOOTH, a, s))) return r;

@@ -263,6 +263,124 @@ __global__ __launch_bounds__(NT) void k_mg_resid_restrict(const double* __restri
     }
 }
 
+// The two legs of a 2D grid's visit, a launch each: a workgroup takes 32 x 8 cells and recomputes what its
+// sweeps read beyond them (the first sweep on two cells around, the second on one), in LDS. Bound by launches
+// and load latency on all grids but the largest: a launch is about 4 us whatever it does, and the legs were two
+// launches each. 512 x 256 Grad_Q 2.00 -> 1.62 ms, eight cases' CAC steps 5.57 -> 4.97 ms, a hierarchy's 21.4 ->
+// 19.6 ms. The arithmetic is k_mg_smooth's and k_mg_resid_restrict's.
+constexpr int MGX = 32, MGY = 8;
+static_assert(MGX * MGY == NT, "a cell a thread");
+
+// coordinate i of direction d taken into the domain across a periodic side; false: no such cell
+__device__ __forceinline__ bool mg_wrap(const MgGrid& G, int d, int& i)
+{
+    const int n = G.n[d];
+    if (G.periodic[d]) i = (i < 0) ? i + n : (i >= n) ? i - n : i;
+    return i >= 0 && i < n;
+}
+
+// mg_apply at cell (i,j) on values in LDS rows of W, x at the cell's
+template <int W>
+__device__ __forceinline__ double mg_apply_lds(const MgGrid& G, const double* x, const double* __restrict__ b0,
+                                               const double* __restrict__ b1, int i, int j)
+{
+    const double xc = x[0];
+    double acc = 0.0, flo = 0.0, fhi = 0.0;
+    if (i > 0 || G.periodic[0]) flo = b0[mg_face(G, 0, i, j, 0)] * (xc - x[-1]);
+    if (i < G.n[0] - 1 || G.periodic[0]) fhi = b0[mg_face(G, 0, i + 1, j, 0)] * (x[1] - xc);
+    acc += (flo - fhi) * G.ih2[0];
+    flo = fhi = 0.0;
+    if (j > 0 || G.periodic[1]) flo = b1[mg_face(G, 1, i, j, 0)] * (xc - x[-W]);
+    if (j < G.n[1] - 1 || G.periodic[1]) fhi = b1[mg_face(G, 1, i, j + 1, 0)] * (x[W] - xc);
+    acc += (flo - fhi) * G.ih2[1];
+    return acc;
+}
+
+// the sweep's start on the tile and two cells around (rows of MGX + 4), then one sweep on the tile and one cell
+// around (rows of MGX + 2)
+template <typename V>
+__device__ __forceinline__ void mg_tile_sweep(const MgGrid& G, int i0, int j0, double* s0, double* s1, const V& value,
+                                              const double* __restrict__ r, const double* __restrict__ id,
+                                              const double* __restrict__ b0, const double* __restrict__ b1, double omega)
+{
+    for (int q = threadIdx.x; q < (MGX + 4) * (MGY + 4); q += NT) {
+        int i = i0 - 2 + q % (MGX + 4), j = j0 - 2 + q / (MGX + 4);
+        if (mg_wrap(G, 0, i) && mg_wrap(G, 1, j)) s0[q] = value(i, j);
+    }
+    __syncthreads();
+    for (int q = threadIdx.x; q < (MGX + 2) * (MGY + 2); q += NT) {
+        const int li = q % (MGX + 2), lj = q / (MGX + 2);
+        int i = i0 - 1 + li, j = j0 - 1 + lj;
+        if (!mg_wrap(G, 0, i) || !mg_wrap(G, 1, j)) continue;
+        const double* x = s0 + (lj + 1) * (MGX + 4) + li + 1;
+        const long long c = mg_idx(G, i, j, 0);
+        s1[q] = x[0] + omega * id[c] * (r[c] - mg_apply_lds<MGX + 4>(G, x, b0, b1, i, j));
+    }
+    __syncthreads();
+}
+
+__device__ __forceinline__ void mg_tile(const MgGrid& G, int& i0, int& j0)
+{
+    const int ntx = (G.n[0] + MGX - 1) / MGX, t = blockIdx.x;
+    j0 = (t / ntx) * MGY;
+    i0 = (t % ntx) * MGX;
+}
+
+__global__ __launch_bounds__(NT) void k_mg_down(const double* __restrict__ sc, double* __restrict__ y,
+                                                const double* __restrict__ r, const double* __restrict__ b0,
+                                                const double* __restrict__ b1, const double* __restrict__ id, MgGrid G,
+                                                double omega, double* __restrict__ rc, MgGrid Gc)
+{
+    if (sc && sc[CG_DONE] != 0.0) return;
+    __shared__ double s0[(MGX + 4) * (MGY + 4)], s1[(MGX + 2) * (MGY + 2)], res[MGX * MGY];
+    int i0, j0;
+    mg_tile(G, i0, j0);
+    auto value = [&](int i, int j) __attribute__((always_inline)) -> double {
+#pragma clang fp contract(off)
+        const long long c = mg_idx(G, i, j, 0);
+        return omega * id[c] * r[c];
+    };
+    mg_tile_sweep(G, i0, j0, s0, s1, value, r, id, b0, b1, omega);
+    const int li = threadIdx.x % MGX, lj = threadIdx.x / MGX, i = i0 + li, j = j0 + lj;
+    if (i < G.n[0] && j < G.n[1]) {
+        const double* x = s1 + (lj + 1) * (MGX + 2) + li + 1;
+        const long long c = mg_idx(G, i, j, 0);
+        y[c] = x[0];
+        res[threadIdx.x] = r[c] - mg_apply_lds<MGX + 2>(G, x, b0, b1, i, j);
+    }
+    __syncthreads();
+    if (threadIdx.x >= NT / 4) return;
+    const int ci = threadIdx.x % (MGX / 2), cj = threadIdx.x / (MGX / 2);
+    if (i0 / 2 + ci >= Gc.n[0] || j0 / 2 + cj >= Gc.n[1]) return;
+    const double* q = res + 2 * cj * MGX + 2 * ci;
+    double s = q[0];
+    s += q[1];
+    s += q[MGX];
+    s += q[MGX + 1];
+    rc[mg_idx(Gc, i0 / 2 + ci, j0 / 2 + cj, 0)] = s * 0.25;
+}
+
+__global__ __launch_bounds__(NT) void k_mg_up(const double* __restrict__ sc, const double* __restrict__ x1,
+                                              double* __restrict__ y, const double* __restrict__ r,
+                                              const double* __restrict__ b0, const double* __restrict__ b1,
+                                              const double* __restrict__ id, MgGrid G, double omega,
+                                              const double* __restrict__ xc, MgGrid Gc)
+{
+    if (sc && sc[CG_DONE] != 0.0) return;
+    __shared__ double s0[(MGX + 4) * (MGY + 4)], s1[(MGX + 2) * (MGY + 2)];
+    int i0, j0;
+    mg_tile(G, i0, j0);
+    auto value = [&](int i, int j) __attribute__((always_inline)) -> double {
+        return x1[mg_idx(G, i, j, 0)] + xc[mg_idx(Gc, i >> 1, j >> 1, 0)];
+    };
+    mg_tile_sweep(G, i0, j0, s0, s1, value, r, id, b0, b1, omega);
+    const int li = threadIdx.x % MGX, lj = threadIdx.x / MGX, i = i0 + li, j = j0 + lj;
+    if (i >= G.n[0] || j >= G.n[1]) return;
+    const double* x = s1 + (lj + 1) * (MGX + 2) + li + 1;
+    const long long c = mg_idx(G, i, j, 0);
+    y[c] = x[0] + omega * id[c] * (r[c] - mg_apply_lds<MGX + 2>(G, x, b0, b1, i, j));
+}
+
 // the coarsest grid: `sweeps` damped Jacobi sweeps from x = 0 in one workgroup (one cell a thread)
 template <int DIM>
 __global__ __launch_bounds__(1024) void k_mg_bottom(const double* __restrict__ sc, const double* __restrict__ r,
@@ -780,6 +898,18 @@ hipError_t launch_mg_dim(int op, const MgArgs& a, hipStream_t s)
         hipLaunchKernelGGL((k_mg_resid_restrict<DIM>), mg_grid(a.Gc.nc), dim3(NT), 0, s, a.sc, a.src, a.r, a.b[0],
                            a.b[1], a.b[2], a.G, a.dst, a.Gc);
         break;
+    case MG_DOWN:
+    case MG_UP: {
+        if (DIM != 2) return hipErrorInvalidValue;
+        const dim3 tiles((unsigned)(((a.G.n[0] + MGX - 1) / MGX) * ((a.G.n[1] + MGY - 1) / MGY)));
+        if (op == MG_DOWN)
+            hipLaunchKernelGGL(k_mg_down, tiles, dim3(NT), 0, s, a.sc, a.dst, a.r, a.b[0], a.b[1], a.id, a.G, a.omega,
+                               a.rw, a.Gc);
+        else
+            hipLaunchKernelGGL(k_mg_up, tiles, dim3(NT), 0, s, a.sc, a.src, a.dst, a.r, a.b[0], a.b[1], a.id, a.G,
+                               a.omega, a.xc, a.Gc);
+        break;
+    }
     case MG_BOTTOM:
         if (a.G.nc > 1024) return hipErrorInvalidValue;
         hipLaunchKernelGGL((k_mg_bottom<DIM>), dim3(1), dim3(1024), 0, s, a.sc, a.r, a.dst, a.b[0], a.b[1], a.b[2],
