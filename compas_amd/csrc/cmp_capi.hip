@@ -1275,8 +1275,22 @@ int cmp_level_pf_setup(cmp_level* L, const cmp_pf_params* pf)
     CMP_TRYP(hipMemcpy(L->d_cmap, cmap.data(), sizeof(cmp::BoxBlock) * cmap.size(), hipMemcpyHostToDevice));
     CMP_TRYP(hipMalloc(&L->d_sc, sizeof(double) * CG_NSC));
     CMP_TRYP(hipMemset(L->d_sc, 0, sizeof(double) * CG_NSC));
-    CMP_TRYP(hipMalloc(&L->d_part, sizeof(double) * 4 * nblk));
-    CMP_TRYP(hipMemset(L->d_part, 0, sizeof(double) * 4 * nblk));
+    // four slots of partial sums: a value a block of cells, or a workgroup of the dense CG
+    long long npart = nblk, cells = 0, dom = 1;
+    for (int b = 0; b < nbox; ++b) {
+        long long n = 1;
+        for (int d = 0; d < dim; ++d) n *= L->boxes[b].hi[d] - L->boxes[b].lo[d] + 1;
+        cells += n;
+    }
+    cmp::MgGrid D{};
+    for (int d = 0; d < 3; ++d) {
+        D.n[d] = (d < dim) ? L->G.domain_hi[d] - L->G.domain_lo[d] + 1 : 1;
+        dom *= D.n[d];
+    }
+    D.nc = dom;
+    if (dom == cells) npart = std::max(npart, (long long)cmp::mg_parts(dim, D));
+    CMP_TRYP(hipMalloc(&L->d_part, sizeof(double) * 4 * npart));
+    CMP_TRYP(hipMemset(L->d_part, 0, sizeof(double) * 4 * npart));
     if (pf->mechanism == CMP_PF_CAC) {
         CMP_TRYP(hipMalloc(&L->d_Mk, sizeof(double) * na));
         CMP_TRYP(hipMalloc(&L->d_Wk, sizeof(double) * na));
@@ -1428,7 +1442,7 @@ static int mg_sums(const cmp_level* L, const double* sc, size_t m, double* part,
 // One V-cycle on grid m from its residual r, the result left in x[cur]: two damped Jacobi sweeps
 // (the first from zero), the residual restricted, the coarser grid's V-cycle prolonged and added,
 // two more sweeps; the coarsest grid takes its fixed number of sweeps in one workgroup. part non-null: the
-// partials of r.z, z and r (z the result) into part's second to fourth slots of mg_blocks values.
+// partials of r.z, z and r (z the result) into part's second to fourth slots of mg_parts values.
 int cmp::mg_vcycle(cmp_level* L, const double* sc, size_t m, hipStream_t s, double* part)
 {
     const int dim = L->P.dim;
@@ -1492,9 +1506,10 @@ int cmp::mg_vcycle(cmp_level* L, const double* sc, size_t m, hipStream_t s, doub
         a.src = V.x[1];
         a.xc = C.x[C.cur];
         a.dst = V.x[0];
+        a.part = part;
         if ((r = mg_launch(dim, cmp::MG_UP, a, s))) return r;
         V.cur = 0;
-        return part ? mg_sums(L, sc, m, part, s) : CMP_OK;
+        return CMP_OK;
     }
     a.from = cmp::MG_FROM_ZERO;
     a.dst = V.x[1];
@@ -1522,7 +1537,7 @@ int cmp::mg_vcycle(cmp_level* L, const double* sc, size_t m, hipStream_t s, doub
 // and d_R in turn (it even: from d_Pv into d_R), z = V(r).
 static int mg_cg_iteration(cmp_level* L, int it, int maxit, double inv_n, hipStream_t s)
 {
-    const int dim = L->P.dim, nb = cmp::mg_blocks(L->mg[0].G.nc);
+    const int dim = L->P.dim, nb = cmp::mg_parts(dim, L->mg[0].G);
     double* p = (it & 1) ? L->d_Pv : L->d_R;
     double* pap = L->d_part + nb;   // (beside the first slot, which takes r.r)
     cmp::MgArgs a = mg_args(L, L->d_sc);

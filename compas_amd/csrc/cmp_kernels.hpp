@@ -331,7 +331,7 @@ enum MgOp {
 //   launch; the two sweeps from src plus xc on Gc (dst, another array than src) in one launch;
 //   SCATTER: src (dense G) -> dst (box layout); CG_RZ: partials of r.z, z and r into part's second to
 //   fourth slots, r and dst (= z) in box layout.
-// The iteration of a CG whose vectors are dense on G, mg_blocks(G.nc) partials a slot: SMOOTH with part and
+// The iteration of a CG whose vectors are dense on G, mg_parts(dim, G) partials a slot: SMOOTH and UP with part and
 //   CG_SUMS (src = z): partials of r.z, z and r as CG_RZ's; CG_AP: p (dst) = z' + beta p_old, z' = src -
 //   mean, p_old = r, ap (rw) of it, partials of p.ap; CG_XR: x (dst) += al p (src), r (rw) -= al ap (id),
 //   partials of r.r, p.ap from its partials r (another slot than part); CG_END: the four sums, then the iteration's end (first: the solve's start, r.r known).
@@ -364,6 +364,13 @@ inline int mg_blocks(long long n)
 {
     const long long b = (n + NT - 1) / NT;
     return (int)(b > 65536 ? 65536 : b < 1 ? 1 : b);
+}
+// workgroups of a dense CG iteration's kernels (and so partials of a sum): in 2D the tiles of the V-cycle's legs,
+// the last of which adds up its result's sums
+constexpr int MGX = 32, MGY = 8;
+inline int mg_parts(int dim, const MgGrid& G)
+{
+    return dim == 2 ? ((G.n[0] + MGX - 1) / MGX) * ((G.n[1] + MGY - 1) / MGY) : mg_blocks(G.nc);
 }
 
 template <int DIM>

@@ -268,7 +268,6 @@ __global__ __launch_bounds__(NT) void k_mg_resid_restrict(const double* __restri
 // and load latency on all grids but the largest: a launch is about 4 us whatever it does, and the legs were two
 // launches each. 512 x 256 Grad_Q 2.00 -> 1.62 ms, eight cases' CAC steps 5.57 -> 4.97 ms, a hierarchy's 21.4 ->
 // 19.6 ms. The arithmetic is k_mg_smooth's and k_mg_resid_restrict's.
-constexpr int MGX = 32, MGY = 8;
 static_assert(MGX * MGY == NT, "a cell a thread");
 
 // coordinate i of direction d taken into the domain across a periodic side; false: no such cell
@@ -360,11 +359,13 @@ __global__ __launch_bounds__(NT) void k_mg_down(const double* __restrict__ sc, d
     rc[mg_idx(Gc, i0 / 2 + ci, j0 / 2 + cj, 0)] = s * 0.25;
 }
 
+// SUMS: the partials of r.z, z and r, z the result, into part's second to fourth slots
+template <bool SUMS>
 __global__ __launch_bounds__(NT) void k_mg_up(const double* __restrict__ sc, const double* __restrict__ x1,
                                               double* __restrict__ y, const double* __restrict__ r,
                                               const double* __restrict__ b0, const double* __restrict__ b1,
                                               const double* __restrict__ id, MgGrid G, double omega,
-                                              const double* __restrict__ xc, MgGrid Gc)
+                                              const double* __restrict__ xc, MgGrid Gc, double* part)
 {
     if (sc && sc[CG_DONE] != 0.0) return;
     __shared__ double s0[(MGX + 4) * (MGY + 4)], s1[(MGX + 2) * (MGY + 2)];
@@ -375,10 +376,17 @@ __global__ __launch_bounds__(NT) void k_mg_up(const double* __restrict__ sc, con
     };
     mg_tile_sweep(G, i0, j0, s0, s1, value, r, id, b0, b1, omega);
     const int li = threadIdx.x % MGX, lj = threadIdx.x / MGX, i = i0 + li, j = j0 + lj;
-    if (i >= G.n[0] || j >= G.n[1]) return;
-    const double* x = s1 + (lj + 1) * (MGX + 2) + li + 1;
-    const long long c = mg_idx(G, i, j, 0);
-    y[c] = x[0] + omega * id[c] * (r[c] - mg_apply_lds<MGX + 2>(G, x, b0, b1, i, j));
+    double w[3] = {0.0, 0.0, 0.0};
+    if (i < G.n[0] && j < G.n[1]) {
+        const double* x = s1 + (lj + 1) * (MGX + 2) + li + 1;
+        const long long c = mg_idx(G, i, j, 0);
+        const double rq = r[c], z = x[0] + omega * id[c] * (rq - mg_apply_lds<MGX + 2>(G, x, b0, b1, i, j));
+        y[c] = z;
+        w[0] = rq * z;
+        w[1] = z;
+        w[2] = rq;
+    }
+    if (SUMS) mg_block_sums(w, part + gridDim.x, gridDim.x, blockIdx.x);
 }
 
 // the coarsest grid: `sweeps` damped Jacobi sweeps from x = 0 in one workgroup (one cell a thread)
@@ -884,7 +892,7 @@ hipError_t launch_mg_dim(int op, const MgArgs& a, hipStream_t s)
     case MG_DIAG:
         hipLaunchKernelGGL((k_mg_diag<DIM>), mg_grid(a.G.nc), dim3(NT), 0, s, a.b[0], a.b[1], a.b[2], a.dst, a.G);
         break;
-    case MG_SMOOTH: {
+    case MG_SMOOTH: if constexpr (DIM == 3) {
         if (a.part && a.from != MG_FROM_X) return hipErrorInvalidValue;
         const auto f = a.part                    ? k_mg_smooth<DIM, MG_FROM_X, true>
                        : a.from == MG_FROM_X    ? k_mg_smooth<DIM, MG_FROM_X, false>
@@ -893,23 +901,22 @@ hipError_t launch_mg_dim(int op, const MgArgs& a, hipStream_t s)
         hipLaunchKernelGGL(f, mg_grid(a.G.nc), dim3(NT), 0, s, a.sc, a.src, a.dst, a.r, a.b[0], a.b[1], a.b[2],
                            a.id, a.G, a.omega, a.xc, a.Gc, a.part);
         break;
-    }
-    case MG_RESID_RESTRICT:
+    } else return hipErrorInvalidValue;
+    case MG_RESID_RESTRICT: if constexpr (DIM == 3) {
         hipLaunchKernelGGL((k_mg_resid_restrict<DIM>), mg_grid(a.Gc.nc), dim3(NT), 0, s, a.sc, a.src, a.r, a.b[0],
                            a.b[1], a.b[2], a.G, a.dst, a.Gc);
         break;
-    case MG_DOWN:
-    case MG_UP: {
-        if (DIM != 2) return hipErrorInvalidValue;
-        const dim3 tiles((unsigned)(((a.G.n[0] + MGX - 1) / MGX) * ((a.G.n[1] + MGY - 1) / MGY)));
-        if (op == MG_DOWN)
-            hipLaunchKernelGGL(k_mg_down, tiles, dim3(NT), 0, s, a.sc, a.dst, a.r, a.b[0], a.b[1], a.id, a.G, a.omega,
-                               a.rw, a.Gc);
-        else
-            hipLaunchKernelGGL(k_mg_up, tiles, dim3(NT), 0, s, a.sc, a.src, a.dst, a.r, a.b[0], a.b[1], a.id, a.G,
-                               a.omega, a.xc, a.Gc);
+    } else return hipErrorInvalidValue;
+    case MG_DOWN: if constexpr (DIM == 2) {
+        hipLaunchKernelGGL(k_mg_down, dim3((unsigned)mg_parts(2, a.G)), dim3(NT), 0, s, a.sc, a.dst, a.r, a.b[0],
+                           a.b[1], a.id, a.G, a.omega, a.rw, a.Gc);
         break;
-    }
+    } else return hipErrorInvalidValue;
+    case MG_UP: if constexpr (DIM == 2) {
+        hipLaunchKernelGGL((a.part ? k_mg_up<true> : k_mg_up<false>), dim3((unsigned)mg_parts(2, a.G)), dim3(NT), 0, s,
+                           a.sc, a.src, a.dst, a.r, a.b[0], a.b[1], a.id, a.G, a.omega, a.xc, a.Gc, a.part);
+        break;
+    } else return hipErrorInvalidValue;
     case MG_BOTTOM:
         if (a.G.nc > 1024) return hipErrorInvalidValue;
         hipLaunchKernelGGL((k_mg_bottom<DIM>), dim3(1), dim3(1024), 0, s, a.sc, a.r, a.dst, a.b[0], a.b[1], a.b[2],
@@ -924,21 +931,21 @@ hipError_t launch_mg_dim(int op, const MgArgs& a, hipStream_t s)
                            a.sc, a.r, a.dst, a.part);
         break;
     case MG_CG_SUMS:
-        hipLaunchKernelGGL(k_dcg_sums, mg_grid(a.G.nc), dim3(NT), 0, s, a.sc, a.r, a.src, a.G.nc, a.part);
+        hipLaunchKernelGGL(k_dcg_sums, dim3((unsigned)mg_parts(DIM, a.G)), dim3(NT), 0, s, a.sc, a.r, a.src, a.G.nc, a.part);
         break;
     case MG_CG_AP:
-        hipLaunchKernelGGL((k_dcg_ap<DIM>), mg_grid(a.G.nc), dim3(NT), 0, s, a.sc, a.src, a.r, a.dst, a.rw, a.b[0],
+        hipLaunchKernelGGL((k_dcg_ap<DIM>), dim3((unsigned)mg_parts(DIM, a.G)), dim3(NT), 0, s, a.sc, a.src, a.r, a.dst, a.rw, a.b[0],
                            a.b[1], a.b[2], a.G, a.g.dx[0], a.g.dx[1], a.g.dx[2], a.inv_n, a.part);
         break;
     case MG_CG_XR: {
-        const int nb = mg_blocks(a.G.nc);
-        hipLaunchKernelGGL(k_dcg_xr, mg_grid(a.G.nc), dim3(NT), 0, s, a.scw, a.dst, a.rw, a.src, a.id, a.G.nc,
+        const int nb = mg_parts(DIM, a.G);
+        hipLaunchKernelGGL(k_dcg_xr, dim3((unsigned)mg_parts(DIM, a.G)), dim3(NT), 0, s, a.scw, a.dst, a.rw, a.src, a.id, a.G.nc,
                            nb <= 1024 ? nb : 0, a.r, a.part);
         break;
     }
     case MG_CG_END:
-        hipLaunchKernelGGL(k_dcg_end, dim3(1), dim3(1024), 0, s, a.scw, a.part, mg_blocks(a.G.nc), a.maxit, a.inv_n,
-                           a.first);
+        hipLaunchKernelGGL(k_dcg_end, dim3(1), dim3(1024), 0, s, a.scw, a.part, mg_parts(DIM, a.G), a.maxit,
+                           a.inv_n, a.first);
         break;
     default:
         return hipErrorInvalidValue;
