@@ -80,7 +80,7 @@ struct AmrPf {
     int ncells = 0, nlinks = 0;
     double vol_total = 0.0;
     long long ncomp = 0;                  // unknowns of the composite solve (cells no finer level covers)
-    double* d_lsum = nullptr;             // per-level sums, 2 per level
+    double* d_lsum = nullptr;             // per-level sums, 4 per level
     unsigned long long* d_bits = nullptr; // [0] max|u|, [1 + l] max|Grad_Q| of level l
     double* h_pin = nullptr;              // pinned host copies
     int cg_iters = 0;
@@ -1027,16 +1027,17 @@ int amr_comp_solve(cmp_amr* A, double* const* out, hipStream_t s0)
     // the composite cells (the operator's null space)
     const double inv_n = (mg && P.ncomp > 0) ? 1.0 / (double)P.ncomp : 0.0;
     int r;
-    // the level sums of nv partial slots from slot slot0 on, and their sum over the levels (one launch)
-    auto sum_levels = [&](int nv, double* dst, const double* scx, int slot0 = 0) -> int {
+    // the level sums of the first nv partial slots, and their sum over the levels (one launch; the third and
+    // fourth, sum z and sum r, go to sc + CG_ZS)
+    auto sum_levels = [&](int nv, double* dst, const double* scx) -> int {
         LevelParts lp{};
         lp.nlev = nlev;
         for (int l = 0; l < nlev; ++l) {
             const cmp_level* L = A->L[l];
-            lp.part[l] = L->d_part + (long long)slot0 * L->nblocks;
+            lp.part[l] = L->d_part;
             lp.nblocks[l] = L->nblocks;
         }
-        CMP_TRY(launch_reduce_levels(lp, nv, P.d_lsum, dst, s, scx));
+        CMP_TRY(launch_reduce_levels(lp, nv, P.d_lsum, dst, s, scx, sc + CG_ZS));
         return CMP_OK;
     };
     // z = R ID (levels above 0, Jacobi) + the level-0 V-cycle of the restricted R/V at every cell's
@@ -1111,8 +1112,7 @@ int amr_comp_solve(cmp_amr* A, double* const* out, hipStream_t s0)
     }
     if (mg && (r = mg_prepare(L0, s))) return r;
     if ((r = precondition(nullptr))) return r;
-    if ((r = sum_levels(2, sc + CG_RR, nullptr))) return r;
-    if ((r = sum_levels(2, sc + CG_ZS, nullptr, 2))) return r;
+    if ((r = sum_levels(4, sc + CG_RR, nullptr))) return r;
     CMP_TRY(launch_cg_start(sc, s, inv_n));
     for (int l = 0; l < nlev; ++l) {
         cmp_level* L = A->L[l];
@@ -1148,8 +1148,7 @@ int amr_comp_solve(cmp_amr* A, double* const* out, hipStream_t s0)
                                      L->d_part, s));
             }
             if ((r = precondition(sc))) return r;
-            if ((r = sum_levels(2, sc + CG_RRNEW, sc))) return r;
-            if (mg && (r = sum_levels(2, sc + CG_ZS, sc, 2))) return r;
+            if ((r = sum_levels(mg ? 4 : 2, sc + CG_RRNEW, sc))) return r;
             for (int l = 0; l < nlev; ++l) {
                 cmp_level* L = A->L[l];
                 CMP_TRY(launch_cg_p(dim, L->pg, L->maxcells, sc, L->d_Z, L->d_Pv, s, inv_n, P.d_mask[l]));
@@ -1255,7 +1254,7 @@ int cmp_amr_pf_setup(cmp_amr* A, const cmp_pf_params* pf)
         CMP_TRYA(hipMemset(a, 0, sizeof(double) * L->na * P.npf));
         CMP_TRYA(hipMemset(ps, 0, sizeof(double) * L->na * P.npf));
     }
-    CMP_TRYA(hipMalloc(&P.d_lsum, sizeof(double) * 2 * AMR_MAX_LEVELS));
+    CMP_TRYA(hipMalloc(&P.d_lsum, sizeof(double) * 4 * AMR_MAX_LEVELS));
     CMP_TRYA(hipMalloc(&P.d_bits, sizeof(unsigned long long) * (1 + AMR_MAX_LEVELS)));
     CMP_TRYA(hipHostMalloc((void**)&P.h_pin, sizeof(double) * (4 + AMR_MAX_LEVELS), hipHostMallocDefault));
 #undef CMP_TRYA

@@ -618,14 +618,14 @@ hipError_t launch_reduce_sums(const double* part, int nblocks, int nvals, double
                               const double* sc = nullptr);
 // The partial sums of every level of a composite solve in one launch: per level the same fixed-order
 // reduction as launch_reduce_sums (into per[l * nvals + v]), then sums[v] = the levels' values added
-// in level order.
+// in level order (values 2 and 3 into sums2[0] and sums2[1]).
 struct LevelParts {
     const double* part[AMR_MAX_LEVELS];
     int nblocks[AMR_MAX_LEVELS];
     int nlev;
 };
 hipError_t launch_reduce_levels(const LevelParts& lp, int nvals, double* per, double* sums, hipStream_t s,
-                                const double* sc = nullptr);
+                                const double* sc = nullptr, double* sums2 = nullptr);
 hipError_t launch_scale(double* p, long long n, double s_, hipStream_t s);
 hipError_t launch_setd(double* p, double v, hipStream_t s);
 hipError_t launch_zero_u64(unsigned long long* p, int n, hipStream_t s);
