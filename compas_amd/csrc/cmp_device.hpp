@@ -306,14 +306,14 @@ __device__ __forceinline__ double weno5_general(double f_mm, double f_m, double 
 // (sum_k t_k g_k) / (sum_k t_k) of one side with t_k = 10 d_k prod_{j != k} I_j^2, as n / S.
 // I1 = 0 (the cell and both neighbours equal, to 1e-162) gives 0: the middle candidate then takes all weight, or every
 // candidate with weight equals the cell's value; S, which may be 0 then, is replaced in its high word alone.
-// `out` is raised to at least WENO_RANGE where S is not in [2^-800, 2^880) (its high word's distance from the
-// lowest one: subnormal products, overflow, NaN), for which n / S means nothing.
-constexpr unsigned WENO_LO = (1023u - 800u) << 20, WENO_RANGE = (800u + 880u) << 20;
+// `out` is raised to at least WENO_HI where n / S means nothing: S >= 2^880, infinite or NaN (also of I1 = 0, where
+// n may be inf * 0) by S's own high word, S < 2^-800 (subnormal products) by its distance from the lowest one.
+constexpr unsigned WENO_LO = (1023u - 800u) << 20, WENO_HI = (1023u + 880u) << 20;
 __device__ __forceinline__ double weno5_side(double n, double S, double I1, unsigned& out)
 {
-    unsigned hi = (unsigned)__double2hiint(S);
-    if (I1 == 0.0) hi = 0x3FF00000u;
-    out = max(out, hi - WENO_LO);
+    const unsigned raw = (unsigned)__double2hiint(S);
+    const unsigned hi = (I1 == 0.0) ? 0x3FF00000u : raw;
+    out = max(max(out, hi - WENO_LO), raw);
     return quot_normal(n, __hiloint2double((int)hi, __double2loint(S)));
 }
 
@@ -368,7 +368,7 @@ __device__ __forceinline__ void weno5_faces(const S& s, double* LW, double* RW)
         // VGPRs (3D), against 113
         __builtin_amdgcn_sched_barrier(0);
     }
-    if (__builtin_expect(out >= WENO_RANGE, 0)) {
+    if (__builtin_expect(out >= WENO_HI, 0)) {
 #pragma unroll
         for (int n = N0; n <= N1; ++n) {
             LW[n] = weno5_general<1>(s(0, n), s(1, n), s(2, n), s(3, n), s(4, n));

@@ -1,10 +1,10 @@
 """The face reconstruction over the whole range of its data: fields whose differences die out by a factor a
 cell (through every magnitude down to zero), steps between constant states (indicators that are exactly
-zero), rounding-level differences and huge or tiny units, where the WENO weights' products leave the double
-range and the general form takes over. GPU right-hand side of one box against the oracle's: everything finite
-and, per variable, within 1e-12 of max |U| c_max / dx, the size of the fluxes it differences (the bar of the
-other right-hand-side tests; rounding differences of a right-hand side are of the fluxes' size, and some of
-these right-hand sides are rounding alone)."""
+zero), rounding-level differences, huge or tiny units and plateaus between jumps of very different size, where
+the WENO weights' products leave the double range and the general form takes over. GPU right-hand side of one
+box against the oracle's: everything finite and, per variable, within 1e-12 of max |U| c_max / dx, the size of
+the fluxes it differences (the bar of the other right-hand-side tests; rounding differences of a right-hand side
+are of the fluxes' size, and some of these right-hand sides are rounding alone)."""
 import numpy as np
 import pytest
 
@@ -15,7 +15,7 @@ from compas_amd.cases import np_prim_to_cons, prim_to_cons
 pytestmark = pytest.mark.gpu
 
 N = 24
-KINDS = ["fringe-3", "fringe-20", "fringe-60", "step", "ramp-end", "noise", "huge", "tiny"]
+KINDS = ["fringe-3", "fringe-20", "fringe-60", "step", "ramp-end", "noise", "huge", "tiny", "plateau"]
 
 
 def _field(kind, nphase, rng):
@@ -39,14 +39,21 @@ def _field(kind, nphase, rng):
     elif kind == "noise":
         p = 1.0 + 2.2e-16 * rng.integers(0, 3, shape)
         a = a * (1.0 + 2.2e-16 * rng.integers(0, 3, shape))
+    elif kind == "plateau":
+        # three equal cells between a jump of 1e55 and one of 1e29: the product of their squares overflows on one
+        # side of the face in the middle while the other side's sums stay in range
+        q = i % 7
+        u = np.where(q == 0, 1e55, np.where(q <= 3, 1e30, 1e30 * (1.0 + 0.3 * rng.uniform(size=shape))))
+        a = np.full(shape, 0.5)
     else:
         s = 1e30 if kind == "huge" else 1e-30
         p = s * s * (1.0 + 0.3 * rng.uniform(size=shape))
         u, v = s * rng.uniform(-0.3, 0.3, shape), s * rng.uniform(-0.3, 0.3, shape)
         a = rng.uniform(0.1, 0.9, shape)
+    rho = 1e-110 if kind == "plateau" else 1.0
     if nphase:
-        return np.stack([a * 1.0, (1 - a) * 0.6 * 0.14, (1 - a) * 0.4 * 5.0, u, v, p, a, (1 - a) * 0.6, (1 - a) * 0.4])
-    return np.stack([a * 1.0, (1 - a) * 10.0, u, v, p, a])
+        return np.stack([a * rho, (1 - a) * 0.6 * 0.14 * rho, (1 - a) * 0.4 * 5.0 * rho, u, v, p, a, (1 - a) * 0.6, (1 - a) * 0.4])
+    return np.stack([a * rho, (1 - a) * 10.0 * rho, u, v, p, a])
 
 
 @pytest.mark.parametrize("scheme,nphase", [("WENO5", 0), ("WENO5B", 0), ("WENO5", 3)])
