@@ -378,9 +378,9 @@ __device__ __forceinline__ void weno5_faces(const S& s, double* LW, double* RW)
 }
 
 // One side at a time, for the N-phase model: face value sum_k w_k f_k. Fast path: with
-// t_k = d_k prod_{j != k} IS_j^2 the value is (sum_k t_k f_k) / sum_k t_k, taken when that sum lies well inside
-// the double range (no scaling, one division); constant data (all IS zero), extreme IS ratios, NaN and inf go
-// through weno5_weights.
+// t_k = d_k prod_{j != k} IS_j^2 the value is (sum_k t_k f_k) / sum_k t_k, taken when that sum lies so far inside
+// the double range that its product with a face value does too (no scaling, one division); constant data (all IS
+// zero), extreme IS ratios, NaN and inf go through weno5_weights.
 template <int FACE>
 __device__ __forceinline__ double weno5(double f_mm, double f_m, double f_c, double f_p, double f_pp)
 {
@@ -392,7 +392,7 @@ __device__ __forceinline__ double weno5(double f_mm, double f_m, double f_c, dou
     const double q01 = IS[0] * IS[1], q02 = IS[0] * IS[2], q12 = IS[1] * IS[2];
     const double t0 = d0 * (q12 * q12), t1 = d1 * (q02 * q02), t2 = d2 * (q01 * q01);
     const double S = (t0 + t1) + t2;
-    if (S > 1e-290 && S < 1e290) return quot_normal(t0 * f[0] + t1 * f[1] + t2 * f[2], S);
+    if (S > 1e-200 && S < 1e200) return quot_normal(t0 * f[0] + t1 * f[1] + t2 * f[2], S);
     double w[3];
     weno5_weights<FACE>(IS, w);
     return w[0] * f[0] + w[1] * f[1] + w[2] * f[2];

@@ -55,11 +55,13 @@ def _stencils(rng, n):
 
 # 2^133 is 1e40, where the products of four indicators leave the double range from above
 @pytest.mark.parametrize("power", [-400, -140, -60, 0, 60, 110, 127, 133, 150, 200, 400, 500])
-@pytest.mark.parametrize("form", ["host_weno5_faces"])
+@pytest.mark.parametrize("form", ["host_weno5_faces", "host_weno5"])
 def test_weno5_over_the_exponents(dev, form, power):
     """WENO5 has no scale of its own: the face states of 2^p v are 2^p times those of v. Reference: the ratio
     form at unit size. The bound: about 40 roundings of numbers up to 8 max |v| in the indicators, the weights and
     the sum, each indicator's relative error amplified up to 8 times by its cancellation and doubled by its square."""
+    if form == "host_weno5" and abs(power) > 450:
+        pytest.skip("its indicators are not scaled: they leave the double range, as the ratio form's do")
     dev.errors(2.0 ** -25, 2.0 ** -25)
     v = _stencils(np.random.default_rng(11), 200)
     L, R = dev(form, v * 2.0 ** power, out=2)
