@@ -768,8 +768,11 @@ __device__ __forceinline__ void np_mix(const KParams& kp, const double* alpha, c
 }
 
 // Conservative2Primitive (…Conservative2Primitive_Compressible5Eq_NPhase.H:16-60), 1/rho and 1/AP
-// from one division.
-template <int DIM, int NP>
+// from one division. SHORT: by quot, which pays only where the Phase-Field stage stages cells (64^3 two-phase
+// Godunov 22.1 -> 21.3 us a right-hand side). Inside the limiter quot holds 8 VGPRs more at the kernel's peak, a
+// wave less a SIMD (three steps of 700^2 on one card, three-phase MUSCL 0.73 -> 0.94 ms; the Phase-Field
+// right-hand side of 512^2 41 -> 54 us); in the flow's staging three-phase 60^3 MUSCL loses 3%.
+template <int DIM, int NP, bool SHORT = false>
 __device__ __forceinline__ void np_cons2prim(const KParams& kp, const double* U, double* W, int& bad)
 {
     using I = NpIdx<DIM, NP>;
@@ -779,7 +782,7 @@ __device__ __forceinline__ void np_cons2prim(const KParams& kp, const double* U,
     if (rho <= 0.0) bad = CMP_ERR_DENSITY;
     double AP, BP, rho_D;
     np_mix<NP>(kp, U + I::A, U, AP, BP, rho_D, bad);
-    const double inv = quot(1.0, rho * AP);
+    const double inv = SHORT ? quot(1.0, rho * AP) : 1.0 / (rho * AP);
     const double ir = AP * inv;
     double ke = 0.0;
 #pragma unroll
@@ -900,8 +903,9 @@ __device__ __forceinline__ void np_limiter_consistent(const double* s, double* t
 // FVM_Reconstruction2Face_Conservative_LimiterConsistent (…LimiterConsistent_Compressible5Eq_NPhase.H:15-73)
 // on a primitive face state W of the side whose cell primitives are c(n): prim->cons->prim as the
 // reference takes it, the alpha_k rho_k and alpha_k slopes to the face, theta from the alpha slopes,
-// the linear face values with theta times the slope.
-template <int DIM, int NP, typename C>
+// the linear face values with theta times the slope. SHORT: the slopes' quotients by one shared reciprocal (see
+// np_recon_face).
+template <int DIM, int NP, bool SHORT, typename C>
 __device__ __forceinline__ void np_limit_face(const KParams& kp, double* W, const C& c, double dx, int face,
                                               int& bad)
 {
@@ -909,12 +913,12 @@ __device__ __forceinline__ void np_limit_face(const KParams& kp, double* W, cons
     double U[I::N], AP, BP, rho;
     np_prim2cons<DIM, NP>(kp, W, U, AP, BP, rho, bad);
     np_cons2prim<DIM, NP>(kp, U, W, bad);
-    const double h = double(face) * 0.5 * dx, rh = rcp_refined(h);
+    const double h = double(face) * 0.5 * dx, rh = SHORT ? rcp_refined(h) : 0.0;
     double sr[NP], sa[NP], th[NP];
 #pragma unroll
     for (int k = 0; k < NP; ++k) {
-        sr[k] = quot_by(W[k] - c(k), h, rh);
-        sa[k] = quot_by(W[I::A + k] - c(I::A + k), h, rh);
+        sr[k] = SHORT ? quot_by(W[k] - c(k), h, rh) : (W[k] - c(k)) / h;
+        sa[k] = SHORT ? quot_by(W[I::A + k] - c(I::A + k), h, rh) : (W[I::A + k] - c(I::A + k)) / h;
     }
     np_limiter_consistent<NP>(sa, th);
 #pragma unroll
@@ -947,7 +951,7 @@ __device__ __forceinline__ double np_hllc_half(const FaceSideN<DIM, NP>& s, int 
     using I = NpIdx<DIM, NP>;
     const double V = pick<DIM>(s.W + I::MOM, dir);
     const double p = s.W[I::E];
-    const double inv = quot(1.0, S - S_Star);
+    const double inv = 1.0 / (S - S_Star);
     const double q = (S - V) * inv;
 #pragma unroll
     for (int k = 0; k < NP; ++k) {
@@ -969,7 +973,9 @@ __device__ __forceinline__ double np_hllc_half(const FaceSideN<DIM, NP>& s, int 
     return V + Sb * (q - 1.0);
 }
 
-// HLLC (RIEMANN 2) or HLL (1, Riemann_HLL …NPhase.H) of the N-phase model; returns u*_n.
+// HLLC (RIEMANN 2) or HLL (1, Riemann_HLL …NPhase.H) of the N-phase model; returns u*_n. IEEE divisions and
+// roots: the short ones gain nothing here and take two-phase Godunov with HLL from 95 to 98 VGPRs, five waves a SIMD
+// to four (three steps of 700^2 0.333 -> 0.371 ms).
 template <int DIM, int RIEMANN, int NP>
 __device__ __forceinline__ double np_riemann(const FaceSideN<DIM, NP>& L, const FaceSideN<DIM, NP>& R, int dir,
                                              double* F, double& cmax)
@@ -983,15 +989,15 @@ __device__ __forceinline__ double np_riemann(const FaceSideN<DIM, NP>& L, const 
         qL = (m == 0) ? L.W[I::MOM] * L.W[I::MOM] : qL + L.W[I::MOM + m] * L.W[I::MOM + m];
         qR = (m == 0) ? R.W[I::MOM] * R.W[I::MOM] : qR + R.W[I::MOM + m] * R.W[I::MOM + m];
     }
-    cmax = smax(L.c + sqrt_fast(qL), R.c + sqrt_fast(qR));
+    cmax = smax(L.c + sqrt(qL), R.c + sqrt(qR));
     const double pL = L.W[I::E], pR = R.W[I::E];
     if (RIEMANN == 2) {
         const double V_avg = 0.5 * (VL + VR);
         const double c_avg = 0.5 * (L.c + R.c);
         const double SL = smin(V_avg - c_avg, VL - L.c);
         const double SR = smax(V_avg + c_avg, VR + R.c);
-        const double S_Star = quot(pR - pL + L.rho * VL * (SL - VL) - R.rho * VR * (SR - VR),
-                                   L.rho * (SL - VL) - R.rho * (SR - VR));
+        const double S_Star = (pR - pL + L.rho * VL * (SL - VL) - R.rho * VR * (SR - VR))
+                            / (L.rho * (SL - VL) - R.rho * (SR - VR));
         if (S_Star > 0.0) return np_hllc_half<DIM, NP>(L, dir, SL, smin(0.0, SL), S_Star, F);
         if (S_Star < 0.0) return np_hllc_half<DIM, NP>(R, dir, SR, smax(0.0, SR), S_Star, F);
         double FR_[N];
@@ -1003,7 +1009,7 @@ __device__ __forceinline__ double np_riemann(const FaceSideN<DIM, NP>& L, const 
     } else {
         const double Sp = smax(smax(0.0, VL + L.c), VR + R.c);
         const double Sm = smin(smin(0.0, VL - L.c), VR - R.c);
-        const double inv = quot(1.0, Sp - Sm);
+        const double inv = 1.0 / (Sp - Sm);
 #pragma unroll
         for (int n = 0; n < N; ++n) {
             double FL, FR;
@@ -1021,13 +1027,16 @@ __device__ __forceinline__ double np_riemann(const FaceSideN<DIM, NP>& L, const 
 
 // Primitive face states of the N-phase model (FVM_Reconstruction2FaceLR_Conservative_K …NPhase):
 // WENO5 or MUSCL per primitive, then the consistent limiter; Godunov without it. s(t, n) as in
-// face_flux.
+// face_flux. The limiter's slopes take the short quotient but for two-phase MUSCL in 2D, whose kernel it takes
+// from 126 to 130 VGPRs, from four waves a SIMD to three (three steps of 700^2 0.544 -> 0.600 ms); with it 3D gains
+// 2%, WENO5 3%, three phases 4%.
 template <int DIM, int SCHEME, int NP, typename S>
 __device__ __forceinline__ void np_recon_face(const KParams& kp, int limiter, int dir, const S& s, double* LW,
                                               double* RW, int& bad)
 {
     constexpr int N = NpIdx<DIM, NP>::N;
     const double dx = pick<DIM>(kp.dx, dir), idx = pick<DIM>(kp.inv_dx, dir);
+    constexpr bool SHORT = SCHEME == 5 || DIM == 3 || NP == 3;
     if (SCHEME == 5) {
 #pragma unroll
         for (int n = 0; n < N; ++n) {
@@ -1035,16 +1044,16 @@ __device__ __forceinline__ void np_recon_face(const KParams& kp, int limiter, in
             LW[n] = weno5<1>(v0, v1, v2, v3, v4);
             RW[n] = weno5<-1>(v1, v2, v3, v4, v5);
         }
-        np_limit_face<DIM, NP>(kp, LW, [&](int n) { return s(2, n); }, dx, 1, bad);
-        np_limit_face<DIM, NP>(kp, RW, [&](int n) { return s(3, n); }, dx, -1, bad);
+        np_limit_face<DIM, NP, SHORT>(kp, LW, [&](int n) { return s(2, n); }, dx, 1, bad);
+        np_limit_face<DIM, NP, SHORT>(kp, RW, [&](int n) { return s(3, n); }, dx, -1, bad);
     } else if (SCHEME == 1) {
 #pragma unroll
         for (int n = 0; n < N; ++n) {
             LW[n] = muscl(s(0, n), s(1, n), s(2, n), dx, idx, 1, limiter);
             RW[n] = muscl(s(1, n), s(2, n), s(3, n), dx, idx, -1, limiter);
         }
-        np_limit_face<DIM, NP>(kp, LW, [&](int n) { return s(1, n); }, dx, 1, bad);
-        np_limit_face<DIM, NP>(kp, RW, [&](int n) { return s(2, n); }, dx, -1, bad);
+        np_limit_face<DIM, NP, SHORT>(kp, LW, [&](int n) { return s(1, n); }, dx, 1, bad);
+        np_limit_face<DIM, NP, SHORT>(kp, RW, [&](int n) { return s(2, n); }, dx, -1, bad);
     } else {
 #pragma unroll
         for (int n = 0; n < N; ++n) {

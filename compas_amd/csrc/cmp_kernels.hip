@@ -302,7 +302,7 @@ __device__ __forceinline__ void load_cell(const CellSrc& src, double* Uc)
 #pragma unroll
     for (int q = 0; q < N; ++q) Uc[q] = src.p[q * src.sn];
 }
-template <int DIM, int NP>
+template <int DIM, int NP, bool SHORT = false>
 __device__ __forceinline__ void stage_cell(const KParams& kp, double* Uc, unsigned flip, double* slot, int stride, int& bad)
 {
     constexpr int N = NP ? 2 * NP + DIM + 1 : 4 + DIM;
@@ -312,7 +312,7 @@ __device__ __forceinline__ void stage_cell(const KParams& kp, double* Uc, unsign
     for (int m = 0; m < DIM; ++m)
         if ((flip >> m) & 1u) Uc[MOM + m] = -Uc[MOM + m];
     if constexpr (NP > 0)
-        np_cons2prim<DIM, (NP > 0 ? NP : 2)>(kp, Uc, Wc, bad);
+        np_cons2prim<DIM, (NP > 0 ? NP : 2), SHORT>(kp, Uc, Wc, bad);
     else
         cons2prim<DIM>(kp, Uc, Wc, bad);
 #pragma unroll
@@ -427,7 +427,7 @@ __device__ __forceinline__ void dir_pass(const StageCtx<DIM>& cx_, const SH& sh,
                                                 cx_.tlo[2] + z - (D == 2 ? G : 0), bad);
         double Uc[N];
         load_cell<DIM, NP>(src, Uc);
-        stage_cell<DIM, NP>(kp, Uc, src.flip, sW + r, RMAX, bad);
+        stage_cell<DIM, NP, (RIEMANN >= RIEMANN_PF_MIX)>(kp, Uc, src.flip, sW + r, RMAX, bad);
     }
     __syncthreads();
     // 2. faces along D: one face per thread and pass (the fixed shape has at most NT faces per
