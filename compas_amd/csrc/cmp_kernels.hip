@@ -2498,9 +2498,17 @@ template hipError_t launch_dt_dim<CMP_KERNEL_DIM>(const double*, double*, double
 // the chunk's device counter and, once the chunk is exhausted, moves on to the following chunks.
 // Every workgroup leaves after it has found all 8 chunks exhausted; the last one to leave sets the
 // counters back to zero for the next launch. W: the resident waves per SIMD the register allocation
-// must leave room for (2, or 3 at the price of some register spills: the autotuner measures both).
+// must leave room for (2, or 3 at the price of some register spills: the autotuner measures both), and no more
+// than LDS admits workgroups: asked for three where only two fit (three-phase WENO5 in 3D), the compiler drops the
+// request and takes 257 VGPRs, which leave one (three steps of 64^3 1.54 -> 1.90 ms).
+template <int DIM, int SCHEME, int NP, int W>
+struct ListWaves {
+    static constexpr int BYTES = 8 * lds_doubles<NP ? 2 * NP + DIM + 1 : 4 + DIM, LdsOf<DIM, Stencil<SCHEME>::G, ShapeRT>>();
+    static constexpr int FIT = 160 * 1024 / (BYTES + 64);
+    static constexpr int V = W < FIT ? W : FIT;
+};
 template <int DIM, int SCHEME, int RIEMANN, bool THINC, int NP, int W>
-__global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(W)))
+__global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(ListWaves<DIM, SCHEME, NP, W>::V)))
 void k_stage_list(const ListLevel* __restrict__ levs, const ListTile* __restrict__ tiles, int ntiles, int* ctr,
                   ListCall call, int limiter, int mode, int stage, const double* __restrict__ dtp)
 {

@@ -68,3 +68,9 @@ def test_waves_per_simd(kernels, name, dim, scheme, riemann, thinc, last, waves)
     vgpr = found[0]["vgpr_count"]
     assert 512 // (-(-vgpr // 8) * 8) >= waves, vgpr
     assert found[0]["vgpr_spill_count"] == 0
+
+
+def test_work_list_kernels_keep_two_waves(kernels):
+    """Every work-list kernel leaves room for two workgroups a CU, whatever occupancy it is built for."""
+    lists = {k: v["vgpr_count"] for k, v in kernels.items() if "k_stage_listILi" in k}
+    assert len(lists) >= 48 and max(lists.values()) <= 256
