@@ -916,7 +916,7 @@ struct StagePasses { static constexpr bool on = RIEMANN >= RIEMANN_PF_MIX || NP 
 
 // Minimum resident waves per SIMD the register allocator must leave room for: as many as LDS admits
 // workgroups (four waves each, one a SIMD). The flow in 3D stages 48 to 53 KB: three; in 2D 29 KB: four at 107
-// VGPRs. WENO5B's two-sided limiter wants 200 VGPRs: three waves with 112 bytes of spills measured 0.54 ms for
+// VGPRs. WENO5B's two-sided limiter wants 200 VGPRs: three waves with 80 bytes of spills measured 0.52 ms for
 // five steps of 1024 x 256, two without spills 0.62 ms. The Phase-Field stage is bound by memory and takes 91
 // VGPRs by itself.
 template <int DIM, int SCHEME, int RIEMANN, int NP>
