@@ -924,8 +924,8 @@ struct StageWaves {
     static constexpr int W = StagePasses<RIEMANN, NP>::on ? 2 : (SCHEME == 6 || DIM == 3) ? 3 : 4;
 };
 
-template <int DIM, int SCHEME, int RIEMANN, bool THINC, int NP>
-__global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(StageWaves<DIM, SCHEME, RIEMANN, NP>::W)))
+template <int DIM, int SCHEME, int RIEMANN, bool THINC, int NP, int WAVES = StageWaves<DIM, SCHEME, RIEMANN, NP>::W>
+__global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(WAVES)))
 void k_stage(KParams kp, int limiter, int mode, int stage,
              const TileDev* __restrict__ tiles, int ntiles, const BoxDev* __restrict__ boxes,
              BoxDev sbox, int sntx, int snty, int single,
@@ -1054,8 +1054,8 @@ __device__ __forceinline__ double face_at(const KParams& kp, int limiter, const 
 // registers, face averaging) and as a second GPU path the fused kernel is checked against. cmc
 // (valid cells of the box): the wave speed of the face that is the low face of a cell along DIR,
 // written by the DIR 0 launch and max-combined by the later ones (the reference's per-cell c_max).
-template <int DIM, int SCHEME, int RIEMANN, bool THINC, int DIR>
-__global__ __launch_bounds__(NT)
+template <int DIM, int SCHEME, int RIEMANN, bool THINC, int DIR, int WAVES = 2>
+__global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(WAVES)))
 void k_faces(KParams kp, int limiter, BoxDev bx, const double* __restrict__ U,
              double* __restrict__ flux, double* __restrict__ fluxnc, double* __restrict__ cmc)
 {
@@ -1386,9 +1386,14 @@ static hipError_t stage4(const KParams& kp, int limiter, int mode, int stage, co
         grid = sntiles;
     }
     if (grid <= 0) return hipSuccess;
-    hipLaunchKernelGGL((k_stage<DIM, SCHEME, RIEMANN, THINC, NP>), dim3(grid), dim3(NT), 0, s, kp, limiter,
-                       mode, stage, tiles, ntiles, boxes, sb, sntx, snty, single, Us, Un, Uout, dt,
-                       cmax_bits, err, gq, fuse);
+    auto kernel = k_stage<DIM, SCHEME, RIEMANN, THINC, NP>;
+    // WENO5B with THINC in 2D: where few tiles share a CU their latency counts, and two waves a SIMD without
+    // spills beat three with (one box, us: 300^2 30.5 -> 26.7, 450^2 47.0 -> 43.2, 600^2 = 1520 tiles 64.5 -> 62.7;
+    // but three steps of a level of 1786 tiles 0.65 -> 0.68 ms, one box of 1000^2 142 -> 149 us)
+    if constexpr (DIM == 2 && SCHEME == 6 && THINC)
+        if (grid <= 6 * 256) kernel = k_stage<DIM, SCHEME, RIEMANN, THINC, NP, 2>;
+    hipLaunchKernelGGL(kernel, dim3(grid), dim3(NT), 0, s, kp, limiter, mode, stage, tiles, ntiles, boxes, sb, sntx,
+                       snty, single, Us, Un, Uout, dt, cmax_bits, err, gq, fuse);
     return hipGetLastError();
 }
 
@@ -1399,15 +1404,15 @@ static hipError_t faces4(const KParams& kp, int limiter, const BoxDev& box, int 
     long long F = 1;
     for (int m = 0; m < DIM; ++m) F *= (box.hi[m] - box.lo[m] + 1 + (m == dir ? 1 : 0));
     const int grid = (int)((F + NT - 1) / NT);
-    if (dir == 0)
-        hipLaunchKernelGGL((k_faces<DIM, SCHEME, RIEMANN, THINC, 0>), dim3(grid), dim3(NT), 0, s, kp,
-                           limiter, box, U, flux, fluxnc, cmc);
-    else if (dir == 1)
-        hipLaunchKernelGGL((k_faces<DIM, SCHEME, RIEMANN, THINC, 1>), dim3(grid), dim3(NT), 0, s, kp,
-                           limiter, box, U, flux, fluxnc, cmc);
-    else
-        hipLaunchKernelGGL((k_faces<DIM, SCHEME, RIEMANN, THINC, (DIM == 3 ? 2 : 1)>), dim3(grid),
-                           dim3(NT), 0, s, kp, limiter, box, U, flux, fluxnc, cmc);
+    constexpr int D2 = (DIM == 3) ? 2 : 1;
+    auto kernel = (dir == 0) ? k_faces<DIM, SCHEME, RIEMANN, THINC, 0>
+                             : (dir == 1) ? k_faces<DIM, SCHEME, RIEMANN, THINC, 1> : k_faces<DIM, SCHEME, RIEMANN, THINC, D2>;
+    // WENO5B with THINC in 2D: three waves a SIMD once there are enough blocks for them (both directions' c_max,
+    // us: 1000^2 158 -> 146; 300^2 28.1 -> 30.2)
+    if constexpr (DIM == 2 && SCHEME == 6 && THINC)
+        if (grid > 6 * 256)
+            kernel = (dir == 0) ? k_faces<DIM, SCHEME, RIEMANN, THINC, 0, 3> : k_faces<DIM, SCHEME, RIEMANN, THINC, 1, 3>;
+    hipLaunchKernelGGL(kernel, dim3(grid), dim3(NT), 0, s, kp, limiter, box, U, flux, fluxnc, cmc);
     return hipGetLastError();
 }
 
