@@ -47,3 +47,10 @@ def test_tile_edges(gpu, n, scheme, thinc):
         for v in range(P.nstate):
             scale = max(np.abs(U[v]).max(), 1.3 / cref) * cref / 0.1      # (momentum fluxes: the pressure)
             assert np.abs(got[v] - ref[v]).max() <= 1e-12 * scale, (write, v, np.abs(got[v] - ref[v]).max() / scale)
+
+
+@pytest.mark.parametrize("n", [(768, 480), (784, 480), (1000, 400)])
+def test_weno5b_thinc_on_both_sides_of_its_workgroup_rules(gpu, n):
+    """WENO5B with THINC in 2D: 1536 tiles (the last of the two-wave build), 1568 and 1701 tiles, and face blocks
+    below (1442, 1470) and above (1564) the face kernel's bound."""
+    test_tile_edges(gpu, n, "WENO5B", 1)
