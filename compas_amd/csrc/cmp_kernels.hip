@@ -668,15 +668,14 @@ __device__ __forceinline__ void pass_tile(const KParams& kp, int limiter, int mo
 // ms, without 2.71 -> 2.50.
 // Larger tiles (8x8x4, 16x16 in 7 to 16 waves) measured slower: fewer workgroups a CU, so that their loads and
 // barriers have less arithmetic of others to hide behind, and waves unevenly spread over the SIMDs.
-template <int DIM, int SCHEME, int RIEMANN, bool THINC, int NP>
+template <int DIM, int SCHEME, int RIEMANN, bool THINC>
 __device__ __forceinline__ void flow_tile(const KParams& kp, int limiter, int mode, int stage, const BoxDev& bx,
                                           const int* tlo, const int (&halo)[3][2], const BoxDev* __restrict__ boxes,
                                           const double* __restrict__ Us, const double* Un, double* Uout,
                                           const double* __restrict__ dtp, unsigned long long* cmax_bits, int* err,
                                           const FillDev* __restrict__ fd, double* sWF, double* sA, double* sRed)
 {
-    constexpr int N = NP ? 2 * NP + DIM + 1 : 4 + DIM;
-    constexpr int IA = 3 + DIM;
+    constexpr int N = 4 + DIM, IA = 3 + DIM;
     constexpr int G = Stencil<SCHEME>::G;
     using C = Cross<DIM, G>;
     constexpr int TX = C::TX, TY = C::TY, RND = C::RND;
@@ -722,7 +721,7 @@ __device__ __forceinline__ void flow_tile(const KParams& kp, int limiter, int mo
             split3(r, 2 * G, n1, x, y, z);
             slot[o] = C::B0 + x + 2 * G * (y + TY * z);
             const CellSrc src = cell_source<DIM, 0>(ctx, tlo[0] + (x < G ? x - G : n0 + x - G), tlo[1] + y, tlo[2] + z, bad);
-            load_cell<DIM, NP>(src, Uc[o]);
+            load_cell<DIM, 0>(src, Uc[o]);
             flip[o] = src.flip;
         }
     }
@@ -735,7 +734,7 @@ __device__ __forceinline__ void flow_tile(const KParams& kp, int limiter, int mo
             split3(r, n0, 2 * G, x, y, z);
             slot[o] = C::B1 + x + TX * (y + 2 * G * z);
             const CellSrc src = cell_source<DIM, 1>(ctx, tlo[0] + x, tlo[1] + (y < G ? y - G : n1 + y - G), tlo[2] + z, bad);
-            load_cell<DIM, NP>(src, Uc[o]);
+            load_cell<DIM, 0>(src, Uc[o]);
             flip[o] = src.flip;
         }
     }
@@ -749,14 +748,14 @@ __device__ __forceinline__ void flow_tile(const KParams& kp, int limiter, int mo
             slot[o] = C::B2 + x + TX * (y + TY * z);
             const CellSrc src = cell_source<DIM, (DIM == 3 ? 2 : 1)>(ctx, tlo[0] + x, tlo[1] + y,
                                                                      tlo[2] + (z < G ? z - G : n2 + z - G), bad);
-            load_cell<DIM, NP>(src, Uc[o]);
+            load_cell<DIM, 0>(src, Uc[o]);
             flip[o] = src.flip;
         }
     }
 #pragma unroll
     for (int o = 0; o < IT; ++o) {
         if (slot[o] >= 0) {
-            stage_cell<DIM, NP>(kp, Uc[o], flip[o], sWF + slot[o], C::CELLS, bad);
+            stage_cell<DIM, 0>(kp, Uc[o], flip[o], sWF + slot[o], C::CELLS, bad);
             if constexpr (THINC) mixed |= Uc[o][IA] > kp.thinc_eps && Uc[o][IA] < 1.0 - kp.thinc_eps;
         }
     }
@@ -826,21 +825,17 @@ __device__ __forceinline__ void flow_tile(const KParams& kp, int limiter, int mo
             }
             auto st = [&](int t, int q) -> double { return sWF[q * C::CELLS + at[t]]; };
             double c;
-            if constexpr (NP > 0) {
-                un = np_face_flux<DIM, SCHEME, RIEMANN, (NP > 0 ? NP : 2)>(kp, limiter, d, st, Fl, c, bad);
-            } else {
-                // o_d along d, o_1 and o_2 along the other directions in ascending order
-                const int s0 = (d == 0) ? 1 : ((d == 1) ? C::AX : C::AX * C::AY);
-                const int s1 = (d == 0) ? C::AX : 1, s2 = (d == 2) ? C::AX : C::AX * C::AY;
-                const int ab = (x + 1) + C::AX * ((y + 1) + C::AY * (DIM == 3 ? z + 1 : 0));
-                auto aa = [&](int od, int o1, int o2) -> double { return sA[ab + od * s0 + o1 * s1 + o2 * s2]; };
-                auto normal = [&]() -> double { return face_normal_component<DIM>(kp, d, aa); };
-                double aL = -1.0, aR = -1.0;
-                if constexpr (THINC) {
-                    if (iface) thinc_decide<DIM, G>(kp, st, normal, aL, aR);
-                }
-                un = face_flux_decided<DIM, SCHEME, RIEMANN, THINC>(kp, limiter, d, st, aL, aR, Fl, c, bad);
+            // o_d along d, o_1 and o_2 along the other directions in ascending order
+            const int s0 = (d == 0) ? 1 : ((d == 1) ? C::AX : C::AX * C::AY);
+            const int s1 = (d == 0) ? C::AX : 1, s2 = (d == 2) ? C::AX : C::AX * C::AY;
+            const int ab = (x + 1) + C::AX * ((y + 1) + C::AY * (DIM == 3 ? z + 1 : 0));
+            auto aa = [&](int od, int o1, int o2) -> double { return sA[ab + od * s0 + o1 * s1 + o2 * s2]; };
+            auto normal = [&]() -> double { return face_normal_component<DIM>(kp, d, aa); };
+            double aL = -1.0, aR = -1.0;
+            if constexpr (THINC) {
+                if (iface) thinc_decide<DIM, G>(kp, st, normal, aL, aR);
             }
+            un = face_flux_decided<DIM, SCHEME, RIEMANN, THINC>(kp, limiter, d, st, aL, aR, Fl, c, bad);
             // the high face of the tile's last cells belongs to the next tile (or to none)
             if (a < nd) {
                 if (__builtin_isnan(c)) bad = CMP_ERR_NAN;
@@ -898,8 +893,8 @@ __device__ __forceinline__ void flow_tile(const KParams& kp, int limiter, int mo
             const double v = (sWF[N * C::FACES + fp] - sWF[N * C::FACES + fm]) * idx;
             divu = (d == 0) ? v : divu + v;
         }
-        update_cell<DIM, SCHEME, RIEMANN, NP>(kp, mode, stage, bx, tlo[0] + cx, tlo[1] + cy, tlo[2] + cz, acc, divu, Ub,
-                                              Un, Uout, dtp, bad);
+        update_cell<DIM, SCHEME, RIEMANN, 0>(kp, mode, stage, bx, tlo[0] + cx, tlo[1] + cy, tlo[2] + cz, acc, divu, Ub,
+                                             Un, Uout, dtp, bad);
     }
     if (cmax_bits) reduce_cmax(cmax_loc, cmax_bits, sRed, tid);
     bad = max(bad, bad_state);
@@ -976,8 +971,8 @@ void k_stage(KParams kp, int limiter, int mode, int stage,
         pass_tile<DIM, SCHEME, RIEMANN, THINC, NP>(kp, limiter, mode, stage, bx, tlo, ShapeFixed<DIM>{}, halo, boxes, Us,
                                                    Un, Uout, dtp, cmax_bits, err, gq, fd, sWF, sRed);
     else
-        flow_tile<DIM, SCHEME, RIEMANN, THINC, NP>(kp, limiter, mode, stage, bx, tlo, halo, boxes, Us, Un, Uout, dtp,
-                                                   cmax_bits, err, fd, sWF, sA, sRed);
+        flow_tile<DIM, SCHEME, RIEMANN, THINC>(kp, limiter, mode, stage, bx, tlo, halo, boxes, Us, Un, Uout, dtp,
+                                               cmax_bits, err, fd, sWF, sA, sRed);
 }
 
 // One RK stage of a batch of independent levels: every tile of every admitted case in one launch.
@@ -999,8 +994,8 @@ void k_stage_batch(const KParams* __restrict__ kps, int limiter, int stage, cons
     const int tlo[3] = {td.lo[0], td.lo[1], td.lo[2]};
     const int halo[3][2] = {{td.halo[0][0], td.halo[0][1]}, {td.halo[1][0], td.halo[1][1]},
                             {td.halo[2][0], td.halo[2][1]}};
-    flow_tile<DIM, SCHEME, RIEMANN, false, 0>(kps[cs], limiter, MODE_RK, stage, bx, tlo, halo, boxes, Us, Un, Uout,
-                                              dts + cs, cmax_bits + cs, errs + cs, fds + cs, sWF, nullptr, sRed);
+    flow_tile<DIM, SCHEME, RIEMANN, false>(kps[cs], limiter, MODE_RK, stage, bx, tlo, halo, boxes, Us, Un, Uout,
+                                           dts + cs, cmax_bits + cs, errs + cs, fds + cs, sWF, nullptr, sRed);
 }
 
 #ifndef CMP_LIST_UNIT
