@@ -1488,13 +1488,7 @@ int cmp::mg_vcycle(cmp_level* L, const double* sc, size_t m, hipStream_t s, doub
     a.r = V.r;
     a.id = V.id;
     int r;
-    if (m + 1 == L->mg.size()) {
-        a.dst = V.x[0];
-        a.sweeps = L->mg_bottom_sweeps;
-        V.cur = 0;
-        if ((r = mg_launch(dim, cmp::MG_BOTTOM, a, s))) return r;
-        return part ? mg_sums(L, sc, m, part, s) : CMP_OK;
-    }
+    if (m + 1 == L->mg.size()) return CMP_ERR_UNSUPPORTED;   // (at most 1024 cells: the tail's, always)
     if (dim == 2) {
         // two launches a grid (every extent is even: a coarser grid exists)
         auto& C = L->mg[m + 1];

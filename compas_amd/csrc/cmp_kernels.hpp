@@ -318,7 +318,7 @@ struct MgGrid {
 };
 
 enum MgOp {
-    MG_GATHER_R, MG_SCATTER, MG_GATHER_B, MG_RESTRICT_B, MG_DIAG, MG_SMOOTH, MG_RESID_RESTRICT, MG_DOWN, MG_UP, MG_BOTTOM, MG_CG_RZ,
+    MG_GATHER_R, MG_SCATTER, MG_GATHER_B, MG_RESTRICT_B, MG_DIAG, MG_SMOOTH, MG_RESID_RESTRICT, MG_DOWN, MG_UP, MG_CG_RZ,
     MG_CG_SUMS, MG_CG_AP, MG_CG_XR, MG_CG_END
 };
 
@@ -326,9 +326,8 @@ enum MgOp {
 //   GATHER_R: src (box layout) -> dst (dense G); GATHER_B: src (box face buffer) -> b[d] (dense faces);
 //   RESTRICT_B: b[d] (G) -> bc[d] (Gc); DIAG: b -> dst = 1/diag; SMOOTH: dst = x + omega id (r - A x),
 //   x as `from` says (src, zero swept once, src plus xc on Gc); RESID_RESTRICT: dst (Gc) = mean of the
-//   children of r - A src (G); BOTTOM: dst = `sweeps` Jacobi sweeps from 0 on r (G at most 1024 cells);
-//   DOWN, UP (2D): a grid's two sweeps from zero on r (dst) and RESID_RESTRICT of them (rw, on Gc) in one
-//   launch; the two sweeps from src plus xc on Gc (dst, another array than src) in one launch;
+//   children of r - A src (G); DOWN, UP (2D): a grid's two sweeps from zero on r (dst) and RESID_RESTRICT of
+//   them (rw, on Gc) in one launch; the two sweeps from src plus xc on Gc (dst, another array than src) in one;
 //   SCATTER: src (dense G) -> dst (box layout); CG_RZ: partials of r.z, z and r into part's second to
 //   fourth slots, r and dst (= z) in box layout.
 // The iteration of a CG whose vectors are dense on G, mg_parts(dim, G) partials a slot: SMOOTH and UP with part and
@@ -356,7 +355,6 @@ struct MgArgs {
     int first;
     double omega;
     int from;
-    int sweeps;
 };
 
 // blocks of a dense grid's kernels (and so partials of a sum)

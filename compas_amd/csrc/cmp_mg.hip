@@ -389,37 +389,6 @@ __global__ __launch_bounds__(NT) void k_mg_up(const double* __restrict__ sc, con
     if (SUMS) mg_block_sums(w, part + gridDim.x, gridDim.x, blockIdx.x);
 }
 
-// the coarsest grid: `sweeps` damped Jacobi sweeps from x = 0 in one workgroup (one cell a thread)
-template <int DIM>
-__global__ __launch_bounds__(1024) void k_mg_bottom(const double* __restrict__ sc, const double* __restrict__ r,
-                                                    double* x, const double* __restrict__ b0,
-                                                    const double* __restrict__ b1, const double* __restrict__ b2,
-                                                    const double* __restrict__ id, MgGrid G, double omega,
-                                                    int sweeps)
-{
-    if (sc && sc[CG_DONE] != 0.0) return;
-    __shared__ double xs[2][1024];
-    const double* b[3] = {b0, b1, b2};
-    const long long q = threadIdx.x;
-    const bool on = q < G.nc;
-    int i = 0, j = 0, k = 0;
-    double rq = 0.0, iq = 0.0;
-    if (on) {
-        mg_cell<DIM>(G, q, i, j, k);
-        rq = r[q];
-        iq = id[q];
-        xs[0][q] = omega * iq * rq;
-    }
-    __syncthreads();
-    int cur = 0;
-    for (int s = 1; s < sweeps; ++s) {
-        if (on) xs[1 - cur][q] = xs[cur][q] + omega * iq * (rq - mg_apply<DIM>(G, MgValues{G, xs[cur]}, b, i, j, k));
-        __syncthreads();
-        cur = 1 - cur;
-    }
-    if (on) x[q] = xs[cur][q];
-}
-
 // A cell of a grid with the coefficients its operator row reads, kept in registers over the phases of a
 // visit: (A x)_c = sum_d (b_lo (x_c - x_m) - b_hi (x_p - x_c)) / h_d^2, a Neumann domain face with b = 0.
 template <int DIM>
@@ -917,11 +886,6 @@ hipError_t launch_mg_dim(int op, const MgArgs& a, hipStream_t s)
                            a.sc, a.src, a.dst, a.r, a.b[0], a.b[1], a.id, a.G, a.omega, a.xc, a.Gc, a.part);
         break;
     } else return hipErrorInvalidValue;
-    case MG_BOTTOM:
-        if (a.G.nc > 1024) return hipErrorInvalidValue;
-        hipLaunchKernelGGL((k_mg_bottom<DIM>), dim3(1), dim3(1024), 0, s, a.sc, a.r, a.dst, a.b[0], a.b[1], a.b[2],
-                           a.id, a.G, a.omega, a.sweeps);
-        break;
     case MG_SCATTER:
         hipLaunchKernelGGL((k_mg_scatter<DIM>), cell_grid(a.g.cmap, a.g.ncmap, a.maxcells, a.g.nbox), dim3(NT), 0, s,
                            a.g, a.src, a.dst, a.G);
