@@ -41,11 +41,14 @@ __device__ __forceinline__ double smin(double a, double b) { return (b < a) ? b 
 __device__ __forceinline__ double smax(double a, double b) { return (a < b) ? b : a; }  // std::max
 __device__ __forceinline__ double dsign(double x) { return (x > 0.0) ? 1.0 : ((x < 0.0) ? -1.0 : 0.0); }
 
-// n / d for normal d and results: v_rcp_f64 (relative error 2^-24.4 measured), one Newton step, and the
-// quotient corrected by its own residual, which squares what error is left: equal to the IEEE quotient in
-// 4 million samples over 240 decades, in 6 instructions instead of the 11 of the IEEE sequence (which also
-// rescales subnormal and huge operands). quot: any operands; a denominator outside the range takes the IEEE
-// division, so zero and infinite ones give what they always gave.
+// n / d for normal d and normal, representable quotients: v_rcp_f64 (relative error 2^-24.4 measured), one Newton
+// step (2^-48), and the quotient corrected by its own residual, which squares what error is left: the rounded
+// result is the IEEE quotient unless the exact one lies within 2^-95 of its size of a rounding boundary (2^-41 of
+// all operands; none in 4 million samples over 240 decades here, and tests/test_device_math.py). 6 instructions
+// instead of the 11 of the IEEE sequence, which also rescales subnormal and huge operands. quot: any denominator
+// (one outside the range takes the IEEE division, so zero and infinite ones give what they always gave) under a
+// finite numerator whose quotient is representable; an infinite numerator, or a quotient beyond the double range,
+// gives NaN where IEEE gives infinity.
 __device__ __forceinline__ double rcp_refined(double d)
 {
     const double r = __builtin_amdgcn_rcp(d);
@@ -354,9 +357,9 @@ __device__ __forceinline__ void weno5_pair(double v0, double v1, double v2, doub
 }
 
 // weno5_pair for the primitives N0..N1 of a face (s(t, n): primitive n of stencil cell t), one run of code
-// without branches; a face with a sum out of range is done again by weno5_general (differences below 1e-36
-// or so, ratios of indicators beyond 1e70, NaN and inf: a thin fringe where a disturbance's rounding dies
-// out, and nothing else in ordinary flows).
+// without branches; a face with a sum out of range is done again by weno5_general (differences all below about
+// 1e-30 or above 1e33, ratios of indicators beyond about 1e120, NaN and inf: a thin fringe where a disturbance's
+// rounding dies out, and nothing else in ordinary flows).
 template <int N0, int N1, typename S>
 __device__ __forceinline__ void weno5_faces(const S& s, double* LW, double* RW)
 {

@@ -660,12 +660,12 @@ __device__ __forceinline__ void pass_tile(const KParams& kp, int limiter, int mo
 // The flow stage of one tile (box bx, lowest cell tlo, halo sources halo): the cross of primitives, the faces
 // of every direction in one list, the cell update of `mode`; c_max max-accumulated into *cmax_bits, the error
 // word into *err. sWF / sA / sRed: the workgroup's LDS (sA: THINC only).
-// Bound by FP64 issue (81% of the cycles on a 256^3 level). Against the direction passes above, a 3D tile
+// Bound by VALU issue (83% of a CU's busy cycles on a 256^3 level; 59% of the instructions are FP64 arithmetic). Against the direction passes above, a 3D tile
 // stages 864 cells instead of 1248, waits at 4 barriers instead of 12, and its 688 faces fill 10.75 waves
 // instead of 12; a clipped tile's faces fill as many waves as it has faces. Same boxes, before and after, on
-// one card: ten steps of 256^2 208 -> 190 us, five of 1024 x 256 with WENO5B 694 -> 544, four of a ragged
-// 75 x 61 x 50 level 577 -> 467, 24 served cases 781 -> 675; the 256^3 droplet's stage with THINC 2.94 -> 2.83
-// ms, without 2.71 -> 2.50.
+// one card: ten steps of 256^2 208 -> 195 us, five of 1024 x 256 with WENO5B 694 -> 531 (517 with its limiter's
+// sides apart), four of a ragged 75 x 61 x 50 level 577 -> 462, 24 served cases 781 -> 672; the 256^3 droplet's
+// stage with THINC 2.94 -> 2.83 ms, without 2.71 -> 2.50.
 // Larger tiles (8x8x4, 16x16 in 7 to 16 waves) measured slower: fewer workgroups a CU, so that their loads and
 // barriers have less arithmetic of others to hide behind, and waves unevenly spread over the SIMDs.
 template <int DIM, int SCHEME, int RIEMANN, bool THINC>
@@ -903,9 +903,14 @@ __device__ __forceinline__ void flow_tile(const KParams& kp, int limiter, int mo
 
 // Which stages go direction by direction (pass_tile): the Phase-Field flux, whose tiles mostly have no face to
 // compute and want many small workgroups (256^3 droplet: 0.44 ms a stage, 0.75 ms as a face list), and the
-// N-phase model. Its hierarchies interpolate ghost cells with one slope factor for all components, which turns
-// a state's last bits into 1e-6 of a run's difference after a few steps: it keeps the arithmetic it has, bit
-// for bit (as a face list, in weno5_pair's form, five steps of 512^2 took 0.54 ms against 0.91).
+// N-phase model, for its rounding. A hierarchy interpolates ghost cells with one slope factor for all components,
+// which turns a state's last bits into 1e-6 of a run's difference after a few steps (with the faces in
+// weno5_pair's form one state in 17 of the four-level rings came out 4e-6 from the former result), so the N-phase
+// faces keep the order of their operations; what short divisions they have give IEEE's quotients but for those
+// quot leaves out. A face list of the same operations takes its direction at run time and is contracted
+// differently. One kernel serves hierarchies and single levels, which have no such interpolation and would gain
+// (five steps of 512^2, us: 900 now, 720 as a face list, 586 with weno5_pair's faces). The two-phase hierarchies
+// interpolate the same way and did change by rounding: 5e-14 over the two steps of two levels that are timed.
 template <int RIEMANN, int NP>
 struct StagePasses { static constexpr bool on = RIEMANN >= RIEMANN_PF_MIX || NP > 0; };
 

@@ -204,8 +204,10 @@ __global__ __launch_bounds__(NT) void k_mg_diag(const double* __restrict__ b0, c
 // one damped Jacobi sweep y = x + omega D^-1 (r - A x). FROM: x the array (MG_FROM_X), the sweep from zero
 // omega D^-1 r (MG_FROM_ZERO) or the array plus the coarser grid's value at the parent cell
 // (MG_FROM_COARSE), the last two computed where they are read: a launch and a pass over memory each against
-// one or two more loads a neighbour, all from cache: four launches a grid instead of six. SUMS: the last
-// sweep of a CG's preconditioner adds up r.z, z and r as it goes.
+// one or two more loads a neighbour: four launches a grid instead of six. It pays at all sizes (3D Grad_Q with the
+// two computed in launches of their own / so: 32^3 1.67 / 1.56 ms, 64^3 2.88 / 2.70, 128^3 7.87 / 7.37, 256^3
+// 51.3 / 50.1; before the dense CG and the one-workgroup coarse end 3.22, 4.83, 11.08, 62.2). SUMS: the last sweep
+// of a CG's preconditioner adds up r.z, z and r as it goes.
 template <int DIM, int FROM, bool SUMS>
 __global__ __launch_bounds__(NT) void k_mg_smooth(const double* __restrict__ sc, const double* __restrict__ x,
                                                   double* __restrict__ y, const double* __restrict__ r,

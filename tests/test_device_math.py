@@ -1,5 +1,5 @@
-"""The face arithmetic of compas_amd/csrc/cmp_device.hpp on the host (tests/device_math_host.cpp): WENO5 face
-states against the oracle's ratio form over the exponent range."""
+"""The face arithmetic of compas_amd/csrc/cmp_device.hpp on the host (tests/device_math_host.cpp): the short
+quotient and root against IEEE, WENO5 face states against the oracle's ratio form over the exponent range."""
 import ctypes
 import os
 import subprocess
@@ -31,6 +31,32 @@ def dev(tmp_path_factory):
 
     call.errors = lib.host_errors
     yield call
+
+
+# the hardware's v_rcp_f64 and v_rsq_f64 were measured within 2^-24.4 and 2^-24.2 of the exact values
+@pytest.mark.parametrize("err", [-2.0 ** -24, -2.0 ** -27, 0.0, 2.0 ** -26, 2.0 ** -24])
+def test_short_quotient_and_root_are_ieee(dev, err):
+    """After a Newton step the reciprocal is within 2^-48, the quotient's correction within 2^-95 of it: the
+    rounded result differs from IEEE only where the exact one lies that close to a rounding boundary, 2^-41 of
+    all operands."""
+    dev.errors(err, err)
+    rng = np.random.default_rng(7)
+    n = 200000
+    mant = lambda: rng.uniform(1.0, 2.0, n) * rng.choice([-1.0, 1.0], n)  # noqa: E731
+    d = mant() * 10.0 ** rng.uniform(-289, 289, n)
+    q = mant() * 10.0 ** rng.uniform(-100, 100, n)
+    a = np.where(np.abs(np.log10(np.abs(d)) + np.log10(np.abs(q))) < 290, q, 1.0 / q) * d
+    a = np.where(np.isfinite(a) & (np.abs(a) > 1e-290) & (np.abs(a) < 1e290), a, d)
+    assert (dev("host_quot", a, d) == a / d).all()
+    x = np.abs(d)
+    assert (dev("host_sqrt", x) == np.sqrt(x)).all()
+    # denominators outside the range, and what IEEE division gives for them
+    with np.errstate(all="ignore"):
+        a = np.array([1.0, -1.0, 0.0, 1.0, 1.0, 1e-300, 3.0, np.nan, 1.0])
+        d = np.array([0.0, 0.0, 0.0, np.inf, -np.inf, 1e-300, 5e-324, 1.0, np.nan])
+        np.testing.assert_array_equal(dev("host_quot", a, d), a / d)
+        x = np.array([0.0, np.inf, 5e-324, 1e-300, 1e300, -1.0, np.nan])
+        np.testing.assert_array_equal(dev("host_sqrt", x), np.sqrt(x))
 
 
 def _stencils(rng, n):
