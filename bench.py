@@ -958,7 +958,7 @@ def main():
         scheme = {(1, 5): 5, (1, 6): 6, (0, 0): 0}.get((P.id_weno, P.id_limiter), 1)
         targs = "%d, %d, %d, %s, %d" % (P.dim, scheme, P.id_riemann, "true" if P.id_thinc else "false", P.nphase)
         prefix = ("void cmp::k_stage_list<%s, %d>" % (targs, tiles_waves) if tiles_on
-                  else "void cmp::k_stage<%s>" % targs)
+                  else "void cmp::k_stage<%s, " % targs)   # (then the waves a SIMD it is built for)
         # the counter runs take this run's tile choice from its cache (no sweep of their own)
         import tempfile
         from compas_amd import tile_cache_save
