@@ -288,9 +288,7 @@ __device__ __forceinline__ CellSrc cell_source(const StageCtx<DIM>& cx_, int i, 
     const int cd = (D == 0) ? i : ((D == 1) ? j : k);
     if (cx_.fd && (cd < bx.lo[D] || cd > bx.hi[D]))
         return halo_source<DIM, D>(cx_, cd > bx.hi[D] ? 1 : 0, i, j, k, bad);
-    // (from the tile's first cell a cell of the tile or its layers is a few rows or planes away: 32 bits)
-    const int rel = (i - cx_.tlo[0]) + (int)bx.sj * (j - cx_.tlo[1]) + (int)bx.sk * (k - cx_.tlo[2]);
-    return {cx_.Ut + rel, bx.sn, 0u};
+    return {cx_.Ut + fab_step<DIM>(bx, i - cx_.tlo[0], j - cx_.tlo[1], k - cx_.tlo[2]), bx.sn, 0u};
 }
 
 // A staged cell: its components from their source, then its primitives into its LDS slot (component stride
@@ -704,7 +702,7 @@ __device__ __forceinline__ void flow_tile(const KParams& kp, int limiter, int mo
     int cx, cy, cz;
     split3(tid, n0, n1, cx, cy, cz);
     const bool valid = tid < nc;
-    const unsigned cell = (unsigned)(cx + (int)bx.sj * cy + (int)bx.sk * cz);
+    const unsigned cell = cx + (unsigned)bx.sj * cy + (DIM == 3 ? (unsigned)bx.sk * cz : 0u);   // (cy < 15, cz < 3: below 2^32 in any memory)
     slot[0] = -1;
     flip[0] = 0u;
     if (valid) {

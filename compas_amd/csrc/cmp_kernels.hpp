@@ -54,6 +54,15 @@ __device__ __forceinline__ long long fab_index(const BoxDev& bx, int i, int j, i
     return (long long)(i - bx.flo[0]) + bx.sj * (j - bx.flo[1]) + bx.sk * (k - bx.flo[2]);
 }
 
+// The offset of a cell (di, dj, dk) away from another of its fab: 32-bit strides and distances, 64-bit products
+// (a single box given by a caller may have rows or planes of which a tile's few exceed 2^31 cells).
+template <int DIM>
+__device__ __forceinline__ long long fab_step(const BoxDev& bx, int di, int dj, int dk)
+{
+    const long long ij = di + (long long)(int)bx.sj * dj;
+    return (DIM == 3) ? ij + (long long)(int)bx.sk * dk : ij;
+}
+
 __device__ __forceinline__ double wave_max(double v)
 {
 #pragma unroll

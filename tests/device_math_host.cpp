@@ -1,5 +1,5 @@
-// The scalar device arithmetic of compas_amd/csrc/cmp_device.hpp compiled for the host, for
-// tests/test_device_math.py. The two hardware approximations it starts from are replaced by the exact value
+// The scalar device arithmetic of compas_amd/csrc (cmp_device.hpp, the index helpers of cmp_kernels.hpp) compiled for
+// the host, for tests/test_device_math.py. The two hardware approximations it starts from are replaced by the exact value
 // with a relative error of the caller's, so that their whole error bound can be covered.
 #include <algorithm>
 #include <cmath>
@@ -31,7 +31,11 @@ static double __hiloint2double(int h, int l)
     return d;
 }
 
+static double __shfl_xor(double v, int, int) { return v; }
+static const dim3 blockIdx, threadIdx;
+
 #include "../compas_amd/csrc/cmp_device.hpp"
+#include "../compas_amd/csrc/cmp_kernels.hpp"
 
 extern "C" {
 void host_errors(double rcp, double rsq) { rcp_error = rcp; rsq_error = rsq; }
@@ -50,6 +54,16 @@ void host_weno5_faces(long n, const double* v, double* L, double* R)
         auto s = [&](int t, int) { return v[6 * i + t]; };
         cmp::weno5_faces<0, 0>(s, L + i, R + i);
     }
+}
+// the offset between cells (i, j, k) and (i + d[0], j + d[1], k + d[2]) of a fab with rows of sj and planes of sk
+// cells: by the staging's step, and by the cells' own indices
+void host_fab_step(long long sj, long long sk, const int* c, const int* d, long long* step, long long* index)
+{
+    cmp::BoxDev bx{};
+    bx.sj = sj;
+    bx.sk = sk;
+    *step = sk ? cmp::fab_step<3>(bx, d[0], d[1], d[2]) : cmp::fab_step<2>(bx, d[0], d[1], 0);
+    *index = cmp::fab_index(bx, c[0] + d[0], c[1] + d[1], c[2] + d[2]) - cmp::fab_index(bx, c[0], c[1], c[2]);
 }
 // one side at a time (the N-phase model)
 void host_weno5(long n, const double* v, double* L, double* R)

@@ -29,7 +29,7 @@ def dev(tmp_path_factory):
         getattr(lib, name)(ctypes.c_long(len(a[0])), *[ctypes.c_void_p(x.ctypes.data) for x in a + res])
         return res if out > 1 else res[0]
 
-    call.errors = lib.host_errors
+    call.errors, call.lib = lib.host_errors, lib
     yield call
 
 
@@ -99,3 +99,16 @@ def test_weno5_over_the_exponents(dev, form, power):
     bound = 40 * 8 * 2 * EPS * np.abs(v).max(axis=1)
     assert (np.abs(np.ldexp(L, -power) - rl) <= bound).all()
     assert (np.abs(np.ldexp(R, -power) - rr) <= bound).all()
+
+
+@pytest.mark.parametrize("sj,sk", [(38, 38 * 38), (2 ** 27, 0), (2 ** 28 + 7, 0), (20006, 430000000), (2, 2 ** 30)])
+def test_cells_of_a_tile_of_a_very_large_box(dev, sj, sk):
+    """The staged cells' offsets from their tile's first cell, also where a tile's few rows or planes are more than
+    2^31 cells apart (a 2D box of 2^27 by 15 is 128 GB)."""
+    for d in [(0, 0, 0), (-3, 0, 0), (18, 0, 0), (0, -3, 0), (0, 17, 0), (0, 0, -3), (0, 0, 5), (18, 17, 5)]:
+        if sk == 0 and d[2]:
+            continue
+        step, index = ctypes.c_longlong(), ctypes.c_longlong()
+        dev.lib.host_fab_step(ctypes.c_longlong(sj), ctypes.c_longlong(sk), (ctypes.c_int * 3)(32, 15, 3),
+                              (ctypes.c_int * 3)(*d), ctypes.byref(step), ctypes.byref(index))
+        assert step.value == index.value
